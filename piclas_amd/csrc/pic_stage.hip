@@ -1423,10 +1423,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_MX))
 // (staging writes pw in the place of C_0; a pass with one record per lane
 // forms the four C_k before each batch of 64 is consumed)
 constexpr int kRingCart = 128, kRecCart = 10;
-template <int ALPHA>
+// NW waves of a workgroup share the target: wave wib takes every NW-th source
+// run, and the waves' sums are added in wave order.
+template <int ALPHA, int NW>
 __device__ __attribute__((always_inline)) inline void sf_gather_cart_target(const DevMesh &M, const int32_t *start,
                                                                             const SFArgs &A, double *PS, int t,
-                                                                            double (*L)[kRecCart], int lane) {
+                                                                            double (*L)[kRecCart], int lane, int wib) {
 #pragma clang fp contract(fast)
   constexpr int nd = 64;
   constexpr int kRing = kRingCart, kRec = kRecCart;
@@ -1510,7 +1512,7 @@ __device__ __attribute__((always_inline)) inline void sf_gather_cart_target(cons
       ms0 = start[A.rfirst[qb + lane]]; ms1 = start[A.rend[qb + lane]]; msi = A.rshift[qb + lane];
     }
     const int jn = min(kWave, qend - qb);
-    for (int j = 0; j < jn; ++j) {
+    for (int j = NW > 1 ? wib : 0; j < jn; j += NW) {
       const int s0 = __builtin_amdgcn_readlane(ms0, j), s1 = __builtin_amdgcn_readlane(ms1, j);
       const int si = __builtin_amdgcn_readlane(msi, j);
       const double ox = A.sh[si][0] - bx, oy = A.sh[si][1] - by, oz = A.sh[si][2] - bz;
@@ -1580,6 +1582,21 @@ __device__ __attribute__((always_inline)) inline void sf_gather_cart_target(cons
     for (int g = 0; g < ng; ++g) group(L + (head & (kRing - 1)), g, live);
   }
   const int dofLo = 4 * ((lane >> 2) & 3) + (lane >> 4);
+  if (NW > 1) {   // the rings are done with: they hold the waves' sums
+    double *part = &L[0][0];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int Q = 0; Q < 4; ++Q) part[Q * kWave + lane] = acc[Q];
+    __syncthreads();
+    for (int Q = wib; Q < 4; Q += NW) {
+      const double *p0 = &L[0][0] - (size_t)wib * kRing * kRec + Q * kWave + lane;
+      double sum = p0[0];
+#pragma unroll
+      for (int k = 1; k < NW; ++k) sum += p0[(size_t)k * kRing * kRec];
+      PS[((size_t)t * nd + 16 * Q + dofLo) * 4 + jc] = sum;
+    }
+    return;
+  }
 #pragma unroll
   for (int Q = 0; Q < 4; ++Q) PS[((size_t)t * nd + 16 * Q + dofLo) * 4 + jc] = acc[Q];
 }
@@ -1591,14 +1608,22 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_MX))
   const int lane = lane_id();
   if (!PERSIST) {
     const int t = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x) * (kBlock / kWave) + wib);
-    if (t < M.nElems) sf_gather_cart_target<ALPHA>(M, start, A, PS, t, lds[wib], lane);
+    if (t < M.nElems) sf_gather_cart_target<ALPHA, 1>(M, start, A, PS, t, lds[wib], lane, 0);
     return;
   }
   int range = blockIdx.x & 7;
   for (int t = sf_next_target(A, M.nElems, range, lane); t < M.nElems; t = sf_next_target(A, M.nElems, range, lane)) {
-    sf_gather_cart_target<ALPHA>(M, start, A, PS, t, lds[wib], lane);
+    sf_gather_cart_target<ALPHA, 1>(M, start, A, PS, t, lds[wib], lane, 0);
     __builtin_amdgcn_wave_barrier();
   }
+}
+// one target per workgroup of NW waves, for meshes of too few targets to fill the device
+template <int ALPHA, int NW>
+__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(WPE_MX))) void k_sf_gather_cart_split(DevMesh M, const int32_t *start, SFArgs A, double *PS) {
+  __shared__ double lds[NW][kRingCart][kRecCart];
+  const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int t = xcd_block(blockIdx.x, gridDim.x);
+  if (t < M.nElems) sf_gather_cart_target<ALPHA, NW>(M, start, A, PS, t, lds[wib], lane_id(), wib);
 }
 
 // Mixed-precision shape-function gather for N = 3 on general elements: S and
@@ -2137,6 +2162,23 @@ int emit_scratch_init(int device);
 int set_particles_impl(pic_handle *h, int64_t n, const double *PartState, const int32_t *elem, const int32_t *species,
                        const uint8_t *is_new, bool outsideMarked);
 
+// Waves that share a target of the tensor-grid gather.  One wave per target
+// leaves the device idle below some 10^4 elements (4,096 waves are resident):
+// a step's gather took, in us with 1 / 4 / 8 / 16 waves per target, 1,000
+// elements of 300 particles 486 / 289 / 273 / 296, 512 of 200 315 / 129 /
+// 105 / 113, 216 of 200 315 / 110 / 68 / 59; 4,096 of 200 636 / 613 / 637,
+// 13,824 of 145 1462 / 1395 / 1468 but of 8 148 / 158 (a wave's last batch
+// is padded to 64 records), 110,592 of 200 14736 / 15482.
+// The particle count is the caller's, so the choice, and with it the order
+// of the sums, holds while particles leave.
+int gather_waves(const pic_handle *h) {
+  const int64_t ne = h->hm.nElems;
+  if (ne <= 256) return 16;
+  if (ne <= 2048) return 8;
+  if (ne <= 4096 || (ne <= 16384 && h->nTotal >= 64 * ne)) return 4;
+  return 1;
+}
+
 // the dominant kernel run_deposition launches (PIC_KERNEL_*)
 int deposit_kernel(const pic_handle *h) {
   if (h->par.deposition == PIC_DEPO_NONE) return PIC_KERNEL_NONE;
@@ -2213,11 +2255,27 @@ int run_deposition(pic_handle *h, bool timed) {
           hipLaunchKernelGGL((k_sf_gather_mfma_coop<0, true>), dim3(nblk), dim3(kBlock), 0, h->stream, h->M, h->start, h->sf, h->PS);
         else
           hipLaunchKernelGGL((k_sf_gather_mfma_coop<0, false>), dim3(nblk), dim3(kBlock), 0, h->stream, h->M, h->start, h->sf, h->PS);
-      } else if (h->sf.cartesian && h->sf.alpha == 2)
-        SF_GATHER(k_sf_gather_cart, 2);
-      else if (h->sf.cartesian)
-        SF_GATHER(k_sf_gather_cart, 0);
-      else if (h->sf.alpha == 2 && lin)
+      } else if (h->sf.cartesian) {
+        const int nw = gather_waves(h);
+#define SF_CART(AL)                                                                                          \
+  do {                                                                                                     \
+    if (nw == 16)                                                                                          \
+      hipLaunchKernelGGL((k_sf_gather_cart_split<AL, 16>), dim3(xcd_grid(ne)), dim3(16 * kWave), 0, h->stream, \
+                         h->M, h->start, h->sf, h->PS);                                                    \
+    else if (nw == 8)                                                                                      \
+      hipLaunchKernelGGL((k_sf_gather_cart_split<AL, 8>), dim3(xcd_grid(ne)), dim3(8 * kWave), 0, h->stream, \
+                         h->M, h->start, h->sf, h->PS);                                                    \
+    else if (nw == 4)                                                                                      \
+      hipLaunchKernelGGL((k_sf_gather_cart_split<AL, 4>), dim3(xcd_grid(ne)), dim3(4 * kWave), 0, h->stream, \
+                         h->M, h->start, h->sf, h->PS);                                                    \
+    else                                                                                                   \
+      SF_GATHER(k_sf_gather_cart, AL);                                                                     \
+  } while (0)
+        if (h->sf.alpha == 2) SF_CART(2);
+        else if (h->sf.alpha == 3) SF_CART(3);
+        else SF_CART(0);
+#undef SF_CART
+      } else if (h->sf.alpha == 2 && lin)
         SF_GATHER(k_sf_gather_mfma, 2, true);
       else if (h->sf.alpha == 2)
         SF_GATHER(k_sf_gather_mfma, 2, false);
