@@ -2002,10 +2002,12 @@ struct StepState {       // a stored particle state, sorted by element
 // self-consistent field operator and adjoint buffers
 struct Adjoint {
   double *G = nullptr, *GT = nullptr, *rbar = nullptr, *lrbar = nullptr, *En = nullptr, *lEn = nullptr, *lE = nullptr;
-  double *lx = nullptr, *lv = nullptr, *lF = nullptr, *xi = nullptr;
+  double *lx = nullptr, *lv = nullptr, *lF = nullptr, *xi = nullptr, *lEc = nullptr, *PS = nullptr;
   int32_t *elemNode = nullptr, *nodeOff = nullptr, *nodeInc = nullptr, *srcOff = nullptr, *tgt = nullptr;
   uint8_t *tgtShift = nullptr;
   std::vector<StepState> ck, seg;
+  std::vector<double *> Es;   // fields of the forward steps
+  StepState fin;              // the state after the forward steps
 };
 }  // namespace
 
