@@ -251,21 +251,19 @@ int  pic_adjoint(pic_handle *h, double dt, int32_t K, int32_t checkpoint_every, 
  *              synchronisation between steps; per-stage timers then report the
  *              replays as push/track time)
  *   sf_kernel  0 default, 1 shape-function sums on the vector ALUs, 2 on the
- *              matrix cores (N = 3)
- *   sf_persistent  1: the matrix-core shape-function sums run as persistent
- *              waves, as many as the device holds at once, that take target
- *              elements from atomic counters (one per XCD range of
- *              elements) instead of one wave per target element; for meshes
- *              whose elements hold very different particle counts.  Each
- *              target is summed by one wave in the same order either way, so
- *              the result is bit-identical.
+ *              matrix cores
+ *   sf_persistent  1: on axis-aligned tensor grids (N = 3) of so many elements
+ *              that one wave takes a target element, the shape-function sums
+ *              run as persistent waves, as many as the device holds at once,
+ *              that take target elements from atomic counters (one per XCD
+ *              range of elements).  Elsewhere the waves of a workgroup share
+ *              a target, and this changes nothing.  Each target is summed in
+ *              the same order, so the result is bit-identical.
  *   sf_shared_loads  1: on meshes that are not axis-aligned tensor grids, the
- *              four waves of a workgroup take four consecutive target
- *              elements and stage each record of the union of their source
- *              lists once in LDS for the four (more culls per wave, and no
- *              skipping of the record blocks whose bounding box cannot reach
- *              a target, which the default gather does); bit-identical as
- *              well.  Takes precedence over sf_persistent there. */
+ *              four waves that share a target read every record of its source
+ *              lists, without skipping the blocks of records whose bounding
+ *              box cannot reach it; bit-identical as well.
+ */
 typedef struct {
   int32_t use_graph;
   int32_t sf_kernel;

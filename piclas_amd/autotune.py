@@ -3,8 +3,8 @@
 The stage has a few execution knobs that do not change its results beyond
 round-off in the order of the shape-function sums (pic_set_tuning): graph
 replay of the time step, the shape-function kernel, persistent waves for the
-matrix-core shape-function sums, and record loads shared by the four targets
-of a workgroup (both bit-identical to one wave per target).
+tensor-grid sums, and reading every record block on other meshes (both
+bit-identical to the default).
 ``autotune`` times each candidate on a scratch stage built for the same mesh
 and particles (the caller's stage is not touched) and returns the fastest as
 keyword arguments of ``PICStage.set_tuning``.

@@ -888,8 +888,7 @@ struct SFArgs {
   int alpha;
   int linear;   // NGeo == 1: the barycentre cull is implied by the DOF-box test
   int32_t *work;   // [8] target counters of the persistent gathers (zeroed before each launch)
-  const int32_t *groff, *grfirst, *grend;   // runs of the union of the lists of 4 consecutive targets
-  const uint8_t *grshift;
+  int noSkip;      // read every record block (set per launch)
 };
 
 // record c of a run whose plane starts at the wave-uniform base b: a 32-bit
@@ -1076,22 +1075,32 @@ __device__ inline int sf_next_target(const SFArgs &A, int nE, int &range, int la
 // barycentre, |x|^2/R^2, f vx, f vy, f vz, f): particles that pass the cull
 // are appended, and groups of 4 are consumed once 64 are pending, so groups
 // span source chunks and only the very last group is padded.
+// A target is up to 64 DOFs of an element: all of them for N <= 3 (in NQ
+// quarters of 16), one of its chunks of 64 for higher N.  The waves of a
+// workgroup share the target: wave wib takes every fourth source run, and
+// their sums are added in wave order.
 constexpr int kRingMfma = 128;
-template <int ALPHA, bool LINEAR>
+template <int N> struct GatherShape {
+  static constexpr int nd = (N + 1) * (N + 1) * (N + 1), nch = (nd + kWave - 1) / kWave;
+  static constexpr int NQ = nd >= 48 ? 4 : (nd + 15) / 16;
+};
+template <int N, int ALPHA, bool LINEAR>
 __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(const DevMesh &M, const int32_t *start,
-                                                                            const SFArgs &A, double *PS, int t,
-                                                                            double (*L)[8], int lane) {
+                                                                            const SFArgs &A, double *PS, int tt,
+                                                                            double (*L)[8], int lane, int wib) {
 #pragma clang fp contract(fast)
-  constexpr int nd = 64;
-  constexpr int kRing = kRingMfma;
+  constexpr int nd = GatherShape<N>::nd, nch = GatherShape<N>::nch, NQ = GatherShape<N>::NQ;
+  constexpr int kRing = kRingMfma, NW = kBlock / kWave;
+  const int t = nch == 1 ? tt : tt / nch, d0 = nch == 1 ? 0 : (tt % nch) * kWave;
   const double bx = M.bary[t * 3], by = M.bary[t * 3 + 1], bz = M.bary[t * 3 + 2];
   const double R2i0 = A.r2_sf_inv;
   // operand-side DOF constants, one DOF per quarter:  S = cd - qq + m.q
-  double mx[4], my[4], mz[4], cd[4], acc[4];
+  double mx[NQ], my[NQ], mz[NQ], cd[NQ], acc[NQ];
   double blo[3] = {1e300, 1e300, 1e300}, bhi[3] = {-1e300, -1e300, -1e300};
 #pragma unroll
-  for (int Q = 0; Q < 4; ++Q) {
-    const int d = 16 * Q + (lane & 15);
+  for (int Q = 0; Q < NQ; ++Q) {
+    // (a place past the last DOF repeats that DOF; it is not written)
+    const int d = min(d0 + 16 * Q + (lane & 15), nd - 1);
     const double *xg = M.xGPe + ((size_t)t * nd + d) * 3;
     const double dx = xg[0] - bx, dy = xg[1] - by, dz = xg[2] - bz;
     mx[Q] = 2.0 * R2i0 * dx; my[Q] = 2.0 * R2i0 * dy; mz[Q] = 2.0 * R2i0 * dz;
@@ -1108,7 +1117,7 @@ __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(cons
       bhi[a] = fmax(bhi[a], __shfl_xor(bhi[a], off, kWave));
     }
   // the reference's element cull |x - bary| > r_sf + ElemRadius, compared squared
-  const double thr = A.r_sf + M.radius[t], thr2 = thr * thr;
+  const double thr = A.r_sf + M.radius[t], thr2 = !LINEAR && A.linear ? 1e300 : thr * thr;
   const double R2box = A.r2_sf * (1.0 + 1e-12);
   const double R2skip = R2box * (1.0 + 1e-9), thr2skip = thr2 * (1.0 + 1e-9);
   const int kp = lane >> 4, jc = lane & 3;
@@ -1118,7 +1127,7 @@ __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(cons
     const double qx = rec[0], qy = rec[1], qz = rec[2], qq = rec[3];
     const double bval = rec[4 + jc];
 #pragma unroll
-    for (int Q = 0; Q < 4; ++Q) {
+    for (int Q = 0; Q < NQ; ++Q) {
       const double S = clamp01(mx[Q] * qx + (my[Q] * qy + (mz[Q] * qz + (cd[Q] - qq))));
       double S1 = S * S;
       if (ALPHA == 0) {
@@ -1141,7 +1150,7 @@ __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(cons
       ms0 = start[A.rfirst[qb + lane]]; ms1 = start[A.rend[qb + lane]]; msi = A.rshift[qb + lane];
     }
     const int jn = min(kWave, qend - qb);
-    for (int j = 0; j < jn; ++j) {
+    for (int j = wib; j < jn; j += NW) {
       const int s0 = __builtin_amdgcn_readlane(ms0, j), s1 = __builtin_amdgcn_readlane(ms1, j);
       const int si = __builtin_amdgcn_readlane(msi, j);
       // shifted position (GetPartPosShifted) relative to the target barycentre
@@ -1189,7 +1198,7 @@ __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(cons
       // skip thresholds carry a 1e-9 margin over the cull's for round-off):
       // it is not read.  The blocks of up to 64 at a time are tested one
       // per lane; the kept records are staged in record order, as without
-      // the skip.
+      // the skip (with A.noSkip every block is read).
       const int bfirst = s0 >> 6, blast = s1 > s0 ? (s1 - 1) >> 6 : bfirst - 1;
       for (int wb = bfirst; wb <= blast; wb += kWave) {
         bool reach = false;
@@ -1200,10 +1209,10 @@ __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(cons
           const double gx = fmax(0.0, fmax(blo[0] - hx, lx - bhi[0]));
           const double gy = fmax(0.0, fmax(blo[1] - hy, ly - bhi[1]));
           const double gz = fmax(0.0, fmax(blo[2] - hz, lz - bhi[2]));
-          reach = !(gx * gx + gy * gy + gz * gz > R2skip);
+          reach = A.noSkip || !(gx * gx + gy * gy + gz * gz > R2skip);
           if (!LINEAR) {
             const double nx = fmax(0.0, fmax(lx, -hx)), ny = fmax(0.0, fmax(ly, -hy)), nz = fmax(0.0, fmax(lz, -hz));
-            reach = reach && !(nx * nx + ny * ny + nz * nz > thr2skip);
+            reach = A.noSkip || (reach && !(nx * nx + ny * ny + nz * nz > thr2skip));
           }
         }
         unsigned long long km = __ballot(reach);
@@ -1246,169 +1255,37 @@ __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(cons
     for (int g = 0; g < ng; ++g) group(L + (head & (kRing - 1)), g);
   }
   const int dofLo = 4 * ((lane >> 2) & 3) + (lane >> 4);
+  // the rings are done with: they hold the waves' sums
+  double *part = &L[0][0];
+  __builtin_amdgcn_wave_barrier();
 #pragma unroll
-  for (int Q = 0; Q < 4; ++Q) PS[((size_t)t * nd + 16 * Q + dofLo) * 4 + jc] = acc[Q];
+  for (int Q = 0; Q < NQ; ++Q) part[Q * kWave + lane] = acc[Q];
+  __syncthreads();
+  for (int Q = wib; Q < NQ; Q += NW) {
+    const double *p0 = &L[0][0] - (size_t)wib * kRing * 8 + Q * kWave + lane;
+    double sum = p0[0];
+#pragma unroll
+    for (int k = 1; k < NW; ++k) sum += p0[(size_t)k * kRing * 8];
+    const int d = d0 + 16 * Q + dofLo;
+    if (nd % 64 == 0 || d < nd) PS[((size_t)t * nd + d) * 4 + jc] = sum;
+  }
 }
 
-// One wave per target element (PERSIST false: target from the block index,
-// XCD-contiguous), or persistent waves that take targets from the counters
-// of sf_next_target (PERSIST true: launched at the resident capacity).
-template <int ALPHA, bool LINEAR, bool PERSIST>
+// One target per workgroup, its source runs dealt to the four waves.  With a
+// wave per target the wave of the fullest target ends long after the others
+// on a mesh with uneven occupancy (16 x 64 x 16 annulus, 6 million particles,
+// density e-folding over a tenth of the radius: 5.26 ms, now 3.05; 24 x 96 x
+// 24, 30 million: 15.8 ms, 14.8 as persistent waves, now 13.9), and small
+// meshes leave the device idle (1,000 deformed elements of 200: 335 us, now
+// 247).  Evenly filled large meshes take the same either way (27,000 of 111:
+// 2.69 ms); 16 waves per target are slower everywhere (4.2 and 20.8 ms).
+template <int N, int ALPHA, bool LINEAR>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_MX))) void k_sf_gather_mfma(DevMesh M, const int32_t *start, SFArgs A, double *PS) {
   __shared__ double lds[kBlock / kWave][kRingMfma][8];
-  const int wib = threadIdx.x / kWave;
-  const int lane = lane_id();
-  if (!PERSIST) {
-    const int t = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x) * (kBlock / kWave) + wib);
-    if (t < M.nElems) sf_gather_mfma_target<ALPHA, LINEAR>(M, start, A, PS, t, lds[wib], lane);
-    return;
-  }
-  int range = blockIdx.x & 7;
-  for (int t = sf_next_target(A, M.nElems, range, lane); t < M.nElems; t = sf_next_target(A, M.nElems, range, lane)) {
-    sf_gather_mfma_target<ALPHA, LINEAR>(M, start, A, PS, t, lds[wib], lane);
-    __builtin_amdgcn_wave_barrier();
-  }
-}
-
-// The general gather with the loads shared by a workgroup: its four waves
-// take four consecutive target elements (neighbours that share most of their
-// sources) and walk the union of their lists in chunks of 128 records, staged
-// once in LDS for the four; each wave culls every staged record against its
-// own target.  A target's own records pass its cull in the order of its own
-// runs (a record of an element that is not in its list lies farther than
-// r_sf from its DOF box), so each target's ring, groups and sums are those of
-// k_sf_gather_mfma, bit for bit; the records are read from memory once per
-// workgroup instead of once per wave, for ~1.3x the cull work per wave.
-constexpr int kStageCoop = 128;
-template <int ALPHA, bool LINEAR>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_MX))) void k_sf_gather_mfma_coop(DevMesh M, const int32_t *start, SFArgs A, double *PS) {
-#pragma clang fp contract(fast)
-  constexpr int nd = 64;
-  constexpr int kRing = kRingMfma;
-  __shared__ double lds[kBlock / kWave][kRingMfma][8];
-  __shared__ double4 stg[kStageCoop][2];
-  const int wib = threadIdx.x / kWave;
-  const int lane = lane_id();
-  const int grp = xcd_block(blockIdx.x, gridDim.x);               // block-uniform
-  if (grp * (kBlock / kWave) >= M.nElems) return;                 // blocks of the XCD padding
-  const int t = __builtin_amdgcn_readfirstlane(grp * (kBlock / kWave) + wib);
-  const bool live = t < M.nElems;                                 // wave-uniform
-  const int te = live ? t : 0;
-  double (*L)[8] = lds[wib];
-  const double bx = M.bary[te * 3], by = M.bary[te * 3 + 1], bz = M.bary[te * 3 + 2];
-  const double R2i0 = A.r2_sf_inv;
-  double mx[4], my[4], mz[4], cd[4], acc[4];
-  double blo[3] = {1e300, 1e300, 1e300}, bhi[3] = {-1e300, -1e300, -1e300};
-#pragma unroll
-  for (int Q = 0; Q < 4; ++Q) {
-    const int d = 16 * Q + (lane & 15);
-    const double *xg = M.xGPe + ((size_t)te * nd + d) * 3;
-    const double dx = xg[0] - bx, dy = xg[1] - by, dz = xg[2] - bz;
-    mx[Q] = 2.0 * R2i0 * dx; my[Q] = 2.0 * R2i0 * dy; mz[Q] = 2.0 * R2i0 * dz;
-    cd[Q] = 1.0 - R2i0 * (dx * dx + dy * dy + dz * dz);
-    blo[0] = fmin(blo[0], dx); blo[1] = fmin(blo[1], dy); blo[2] = fmin(blo[2], dz);
-    bhi[0] = fmax(bhi[0], dx); bhi[1] = fmax(bhi[1], dy); bhi[2] = fmax(bhi[2], dz);
-    acc[Q] = 0.0;
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1)
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      blo[a] = fmin(blo[a], __shfl_xor(blo[a], off, kWave));
-      bhi[a] = fmax(bhi[a], __shfl_xor(bhi[a], off, kWave));
-    }
-  const double thr = A.r_sf + M.radius[te], thr2 = thr * thr;
-  const double R2box = A.r2_sf * (1.0 + 1e-12);
-  const int kp = lane >> 4, jc = lane & 3;
-  auto group = [&](const double (*Lh)[8], int g) {
-    const double *rec = Lh[4 * g + kp];
-    const double qx = rec[0], qy = rec[1], qz = rec[2], qq = rec[3];
-    const double bval = rec[4 + jc];
-#pragma unroll
-    for (int Q = 0; Q < 4; ++Q) {
-      const double S = clamp01(mx[Q] * qx + (my[Q] * qy + (mz[Q] * qz + (cd[Q] - qq))));
-      double S1 = S * S;
-      if (ALPHA == 0) {
-        for (int ex = 3; ex <= A.alpha; ++ex) S1 = S * S1;
-      } else {
-#pragma unroll
-        for (int ex = 3; ex <= ALPHA; ++ex) S1 = S * S1;
-      }
-      acc[Q] = __builtin_amdgcn_mfma_f64_4x4x4f64(S1, bval, acc[Q], 0, 0, 0);
-    }
-  };
-  int head = 0, tail = 0;
-  const int q0 = A.groff[grp], qend = A.groff[grp + 1];           // block-uniform
-  for (int qb = q0; qb < qend; qb += kWave) {
-    int ms0 = 0, ms1 = 0, msi = 0;
-    if (qb + lane < qend) {
-      ms0 = start[A.grfirst[qb + lane]]; ms1 = start[A.grend[qb + lane]]; msi = A.grshift[qb + lane];
-    }
-    const int jn = min(kWave, qend - qb);
-    for (int j = 0; j < jn; ++j) {
-      const int s0 = __builtin_amdgcn_readlane(ms0, j), s1 = __builtin_amdgcn_readlane(ms1, j);
-      const int si = __builtin_amdgcn_readlane(msi, j);
-      const double ox = A.sh[si][0] - bx, oy = A.sh[si][1] - by, oz = A.sh[si][2] - bz;
-      const int cnt = s1 - s0;
-      for (int base = 0; base < cnt; base += kStageCoop) {
-        // stage the chunk once for the workgroup (the previous chunk's reads
-        // ended at the barrier below)
-        if (threadIdx.x < kStageCoop && base + int(threadIdx.x) < cnt) {
-          const size_t r = size_t(s0 + base + int(threadIdx.x));
-          stg[threadIdx.x][0] = A.rec[r];
-          stg[threadIdx.x][1] = A.recB[r];
-        }
-        __syncthreads();
-        if (live) {
-          for (int sub = 0; sub < kStageCoop && base + sub < cnt; sub += kWave) {
-            const int k = sub + lane;
-            const bool valid = base + k < cnt;
-            const double4 ra = stg[valid ? k : 0][0], rb = stg[valid ? k : 0][1];
-            const double px = ra.x + ox, py = ra.y + oy, pz = ra.z + oz;
-            const double gx = fmax(0.0, fmax(blo[0] - px, px - bhi[0]));
-            const double gy = fmax(0.0, fmax(blo[1] - py, py - bhi[1]));
-            const double gz = fmax(0.0, fmax(blo[2] - pz, pz - bhi[2]));
-            bool pass = valid && (ra.w != 0.0) && (gx * gx + gy * gy + gz * gz <= R2box);
-            if (!LINEAR) pass = pass && !(px * px + py * py + pz * pz > thr2);
-            const unsigned long long m = __ballot(pass);
-            if (m == 0) continue;
-            if (pass) {
-              double *r = L[(tail + __popcll(m & ((1ull << lane) - 1ull))) & (kRing - 1)];
-              r[0] = px; r[1] = py; r[2] = pz;
-              r[3] = R2i0 * (px * px + py * py + pz * pz);
-              r[4] = rb.x; r[5] = rb.y; r[6] = rb.z; r[7] = rb.w;
-            }
-            tail += __popcll(m);
-            if (tail - head < kWave) continue;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            for (int g = 0; g < kWave / 4; ++g) group(L + (head & (kRing - 1)), g);
-            head += kWave;
-            __builtin_amdgcn_wave_barrier();
-          }
-        }
-        __syncthreads();
-      }
-    }
-  }
-  if (!live) return;
-  const int rest = tail - head;
-  if (rest > 0) {
-    const int ng = (rest + 3) >> 2;
-    if (lane >= rest && lane < 4 * ng) {
-      double *r = L[(head + lane) & (kRing - 1)];
-#pragma unroll
-      for (int c = 0; c < 8; ++c) r[c] = 0.0;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int g = 0; g < ng; ++g) group(L + (head & (kRing - 1)), g);
-  }
-  const int dofLo = 4 * ((lane >> 2) & 3) + (lane >> 4);
-#pragma unroll
-  for (int Q = 0; Q < 4; ++Q) PS[((size_t)t * nd + 16 * Q + dofLo) * 4 + jc] = acc[Q];
+  const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int t = xcd_block(blockIdx.x, gridDim.x);
+  if (t < M.nElems * GatherShape<N>::nch)
+    sf_gather_mfma_target<N, ALPHA, LINEAR>(M, start, A, PS, t, lds[wib], lane_id(), wib);
 }
 
 // The same gather for targets whose Gauss points form an axis-aligned tensor
@@ -2043,7 +1920,7 @@ struct pic_handle {
   bool recFresh = false;  // sf.rec holds the records of the current particle arrays
   bool useGraph = false;  // replay captured two-step graphs in pic_time_step
   bool sfPersist = false; // N = 3 matrix-core gathers: persistent waves that take targets from counters
-  bool sfCoop = false;    // general matrix-core gather: a workgroup's four targets share their record loads
+  bool sfNoSkip = false;  // general matrix-core gather: no record block is skipped
   int nCU = 0;            // compute units of the device
   std::vector<std::pair<const void *, unsigned>> persistGrid;   // resident blocks per persistent kernel
   hipGraph_t graph = nullptr;
@@ -2186,7 +2063,7 @@ int deposit_kernel(const pic_handle *h) {
   if (h->par.deposition == PIC_DEPO_NONE) return PIC_KERNEL_NONE;
   if (h->par.deposition == PIC_DEPO_CVWM) return PIC_KERNEL_CVWM;
   if (h->hm.N == 3 && h->par.precision == PIC_PREC_MIXED) return PIC_KERNEL_SF_MIXED;
-  if (h->hm.N == 3 && h->sfMatrix) return h->sf.cartesian ? PIC_KERNEL_SF_CARTESIAN : PIC_KERNEL_SF_MATRIX;
+  if (h->sfMatrix) return h->sf.cartesian ? PIC_KERNEL_SF_CARTESIAN : PIC_KERNEL_SF_MATRIX;
   return PIC_KERNEL_SF_VALU;
 }
 
@@ -2198,7 +2075,7 @@ int run_deposition(pic_handle *h, bool timed) {
   // ev[8] marks the start of the dominant kernel (after the record pass of the
   // matrix-core gather)
   const bool mixed = h->par.precision == PIC_PREC_MIXED;
-  const bool records = h->par.deposition == PIC_DEPO_SF && N == 3 && (h->sfMatrix || mixed);
+  const bool records = h->par.deposition == PIC_DEPO_SF && (h->sfMatrix || mixed);
   if (timed && !records) HIPCHK(hipEventRecord(h->ev[8], h->stream));
   if (h->par.deposition == PIC_DEPO_NONE) {
     hipLaunchKernelGGL(k_fill_f64, dim3(grid_for(int64_t(nps))), dim3(kBlock), 0, h->stream, h->PS, int64_t(nps));
@@ -2231,61 +2108,54 @@ int run_deposition(pic_handle *h, bool timed) {
         hipLaunchKernelGGL((k_sf_gather_mixed_cart<0>), dim3(nblk), dim3(kBlock), 0, h->stream, h->M, h->start, h->sf, h->PS);
       else
         hipLaunchKernelGGL((k_sf_gather_mixed<0>), dim3(nblk), dim3(kBlock), 0, h->stream, h->M, h->start, h->sf, h->PS);
-    } else if (N == 3 && h->sfMatrix) {
-      const bool lin = h->sf.linear != 0;
-      // persistent waves: the counters start at zero (a fill kernel, which a
-      // captured graph replays), the grid is what the device holds at once
-      if (h->sfPersist)
-        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(kBlock), 0, h->stream, h->sf.work, int64_t(8), 0);
-#define SF_GATHER(K, ...)                                                                                    \
-  do {                                                                                                     \
-    if (h->sfPersist) {                                                                                    \
-      auto kp = K<__VA_ARGS__, true>;                                                                      \
-      hipLaunchKernelGGL(kp, dim3(persist_grid(h, (const void *)kp)), dim3(kBlock), 0, h->stream, h->M,    \
-                         h->start, h->sf, h->PS);                                                          \
-    } else {                                                                                               \
-      auto kp = K<__VA_ARGS__, false>;                                                                     \
-      hipLaunchKernelGGL(kp, dim3(nblk), dim3(kBlock), 0, h->stream, h->M, h->start, h->sf, h->PS);         \
-    }                                                                                                      \
-  } while (0)
-      if (h->sfCoop && !h->sf.cartesian) {
-        if (h->sf.alpha == 2 && lin)
-          hipLaunchKernelGGL((k_sf_gather_mfma_coop<2, true>), dim3(nblk), dim3(kBlock), 0, h->stream, h->M, h->start, h->sf, h->PS);
-        else if (h->sf.alpha == 2)
-          hipLaunchKernelGGL((k_sf_gather_mfma_coop<2, false>), dim3(nblk), dim3(kBlock), 0, h->stream, h->M, h->start, h->sf, h->PS);
-        else if (lin)
-          hipLaunchKernelGGL((k_sf_gather_mfma_coop<0, true>), dim3(nblk), dim3(kBlock), 0, h->stream, h->M, h->start, h->sf, h->PS);
-        else
-          hipLaunchKernelGGL((k_sf_gather_mfma_coop<0, false>), dim3(nblk), dim3(kBlock), 0, h->stream, h->M, h->start, h->sf, h->PS);
-      } else if (h->sf.cartesian) {
+    } else if (h->sfMatrix) {
+      SFArgs a = h->sf;
+      a.noSkip = h->sfNoSkip;
+#define SF_LAUNCH(KERNEL, GRID, BLOCK)                                                                       \
+  hipLaunchKernelGGL((KERNEL), dim3(GRID), dim3(BLOCK), 0, h->stream, h->M, h->start, a, h->PS)
+      if (a.cartesian) {
         const int nw = gather_waves(h);
+        // persistent waves: the counters start at zero (a fill kernel, which a
+        // captured graph replays), the grid is what the device holds at once
+        if (h->sfPersist && nw == 1)
+          hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(kBlock), 0, h->stream, h->sf.work, int64_t(8), 0);
 #define SF_CART(AL)                                                                                          \
   do {                                                                                                     \
-    if (nw == 16)                                                                                          \
-      hipLaunchKernelGGL((k_sf_gather_cart_split<AL, 16>), dim3(xcd_grid(ne)), dim3(16 * kWave), 0, h->stream, \
-                         h->M, h->start, h->sf, h->PS);                                                    \
-    else if (nw == 8)                                                                                      \
-      hipLaunchKernelGGL((k_sf_gather_cart_split<AL, 8>), dim3(xcd_grid(ne)), dim3(8 * kWave), 0, h->stream, \
-                         h->M, h->start, h->sf, h->PS);                                                    \
-    else if (nw == 4)                                                                                      \
-      hipLaunchKernelGGL((k_sf_gather_cart_split<AL, 4>), dim3(xcd_grid(ne)), dim3(4 * kWave), 0, h->stream, \
-                         h->M, h->start, h->sf, h->PS);                                                    \
-    else                                                                                                   \
-      SF_GATHER(k_sf_gather_cart, AL);                                                                     \
+    if (nw == 16) SF_LAUNCH((k_sf_gather_cart_split<AL, 16>), xcd_grid(ne), 16 * kWave);                    \
+    else if (nw == 8) SF_LAUNCH((k_sf_gather_cart_split<AL, 8>), xcd_grid(ne), 8 * kWave);                  \
+    else if (nw == 4) SF_LAUNCH((k_sf_gather_cart_split<AL, 4>), xcd_grid(ne), 4 * kWave);                  \
+    else if (h->sfPersist)                                                                                 \
+      SF_LAUNCH((k_sf_gather_cart<AL, true>), persist_grid(h, (const void *)k_sf_gather_cart<AL, true>), kBlock); \
+    else SF_LAUNCH((k_sf_gather_cart<AL, false>), nblk, kBlock);                                            \
   } while (0)
-        if (h->sf.alpha == 2) SF_CART(2);
-        else if (h->sf.alpha == 3) SF_CART(3);
+        if (a.alpha == 2) SF_CART(2);
+        else if (a.alpha == 3) SF_CART(3);
         else SF_CART(0);
 #undef SF_CART
-      } else if (h->sf.alpha == 2 && lin)
-        SF_GATHER(k_sf_gather_mfma, 2, true);
-      else if (h->sf.alpha == 2)
-        SF_GATHER(k_sf_gather_mfma, 2, false);
-      else if (lin)
-        SF_GATHER(k_sf_gather_mfma, 0, true);
-      else
-        SF_GATHER(k_sf_gather_mfma, 0, false);
-#undef SF_GATHER
+      } else {
+        const unsigned grid = xcd_grid(int64_t(ne) * ((h->hm.nDof + kWave - 1) / kWave));
+#define SF_GENERAL(N, LIN)                                                       \
+  do {                                                                          \
+    if (a.alpha == 2) SF_LAUNCH((k_sf_gather_mfma<N, 2, LIN>), grid, kBlock);    \
+    else if (a.alpha == 3) SF_LAUNCH((k_sf_gather_mfma<N, 3, LIN>), grid, kBlock); \
+    else SF_LAUNCH((k_sf_gather_mfma<N, 0, LIN>), grid, kBlock);                 \
+  } while (0)
+        switch (N) {
+          case 1: SF_GENERAL(1, false); break;
+          case 2: SF_GENERAL(2, false); break;
+          case 3:
+            if (a.linear) SF_GENERAL(3, true);
+            else SF_GENERAL(3, false);
+            break;
+          case 4: SF_GENERAL(4, false); break;
+          case 5: SF_GENERAL(5, false); break;
+          case 6: SF_GENERAL(6, false); break;
+          case 7: SF_GENERAL(7, false); break;
+          default: break;
+        }
+#undef SF_GENERAL
+      }
+#undef SF_LAUNCH
     } else if (h->sf.alpha == 2) {
       LAUNCH_N2(k_sf_gather, N, 2, dim3(nblk), h->M, h->P, h->start, h->sf, h->PS);
     } else {
@@ -2561,10 +2431,6 @@ int pic_create(const pic_mesh_desc *mesh, const pic_params *par, pic_handle **ou
     rc |= upload(h, const_cast<int32_t **>(&h->sf.rfirst), hm.sfRunFirst);
     rc |= upload(h, const_cast<int32_t **>(&h->sf.rend), hm.sfRunEnd);
     rc |= upload(h, const_cast<uint8_t **>(&h->sf.rshift), hm.sfRunShift);
-    rc |= upload(h, const_cast<int32_t **>(&h->sf.groff), hm.sfGrpRunOff);
-    rc |= upload(h, const_cast<int32_t **>(&h->sf.grfirst), hm.sfGrpRunFirst);
-    rc |= upload(h, const_cast<int32_t **>(&h->sf.grend), hm.sfGrpRunEnd);
-    rc |= upload(h, const_cast<uint8_t **>(&h->sf.grshift), hm.sfGrpRunShift);
     for (int s = 0; s < 27; ++s)
       for (int c = 0; c < 3; ++c) h->sf.sh[s][c] = hm.shift[s][c];
     const double a = par->sf_alpha, r = par->sf_radius;
@@ -2612,7 +2478,7 @@ int pic_create(const pic_mesh_desc *mesh, const pic_params *par, pic_handle **ou
     rc |= dalloc(h, &h->P.rx, cap); rc |= dalloc(h, &h->P.ry, cap); rc |= dalloc(h, &h->P.rz, cap);
     rc |= dalloc(h, &h->Q.rx, cap); rc |= dalloc(h, &h->Q.ry, cap); rc |= dalloc(h, &h->Q.rz, cap);
   }
-  if (par->deposition == PIC_DEPO_SF && hm.N == 3) {
+  if (par->deposition == PIC_DEPO_SF) {
     double4 *rec = nullptr;
     rc |= dalloc(h, &rec, size_t(cap) * 2);
     h->sf.rec = rec;
@@ -2936,7 +2802,7 @@ void drop_graph(pic_handle *h) {
 // deposition records of the current arrays, if the gathers read them and
 // the last sort did not write them
 int refresh_records(pic_handle *h) {
-  const bool records = h->par.deposition == PIC_DEPO_SF && h->hm.N == 3 &&
+  const bool records = h->par.deposition == PIC_DEPO_SF &&
                        (h->sfMatrix || h->par.precision == PIC_PREC_MIXED) && h->sf.rec;
   if (!records || h->recFresh) return 0;
   hipLaunchKernelGGL(k_sf_records, dim3(grid_for(std::max<int64_t>(h->n, 1))), dim3(kBlock), 0, h->stream, h->P,
@@ -3021,7 +2887,7 @@ int pic_set_tuning(pic_handle *h, const pic_tuning *t) {
   h->useGraph = t->use_graph != 0;
   if (t->sf_kernel != 0) h->sfMatrix = t->sf_kernel == 2;
   h->sfPersist = t->sf_persistent != 0 && h->sf.work != nullptr;
-  h->sfCoop = t->sf_shared_loads != 0 && h->sf.groff != nullptr;
+  h->sfNoSkip = t->sf_shared_loads != 0;
   return PIC_OK;
 }
 

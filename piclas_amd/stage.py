@@ -456,7 +456,7 @@ class PICStage:
 
     def set_tuning(self, use_graph=False, sf_kernel=0, sf_persistent=False, sf_shared_loads=False):
         """Execution tuning: graph replay of pic_time_step, shape-function kernel (0 default, 1 VALU, 2 matrix),
-        persistent matrix-core shape-function waves, record loads shared by a workgroup's four targets."""
+        persistent waves of the tensor-grid shape-function sums, every record block read on other meshes."""
         t = PicTuning(int(bool(use_graph)), int(sf_kernel), int(bool(sf_persistent)), int(bool(sf_shared_loads)))
         _chk(load_library().pic_set_tuning(self.h, ctypes.byref(t)), "pic_set_tuning")
 
