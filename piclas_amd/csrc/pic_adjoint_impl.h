@@ -659,7 +659,6 @@ int sc_push(pic_handle *h, double dt, const double *E) {
   DevMesh M = h->M;
   M.E = E;
   const dim3 grid(grid_for(std::max<int64_t>(n, 1)));
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(kBlock), 0, h->stream, h->mv.count, int64_t(1), 0);
   if (M.affine && h->hm.N == 3)   // every element affine: xi without Newton
     hipLaunchKernelGGL((k_push_inside<3, false, true>), grid, dim3(kBlock), 0, h->stream, M, h->P, n, dt, h->newElem,
                        h->mv, nDev);

@@ -573,7 +573,7 @@ __global__ __launch_bounds__(kBlock) void k_seg_rank(int nElems, const int32_t *
       if (bin == b) rank[i] = off[b] + __popcll(m & lt);
       off[b] += __popcll(m);
     }
-    if (valid && !st && ne >= 0) rank[i] = atomicAdd(&arrCnt[ne], 1);
+    if (valid && !st && ne >= 0) rank[i] = ~atomicAdd(&arrCnt[ne], 1);   // (negative: an arrival)
   }
   if (lane == 0) stayCnt[w] = stay;
 }
@@ -634,45 +634,40 @@ __global__ __launch_bounds__(1024) void k_scan(int nElems, const int32_t *stayCn
   if (t == 0) newStart[nElems] = carry;
 }
 
-__global__ __launch_bounds__(kBlock) void k_dest(int64_t n, const int32_t *oldElemOf, const int32_t *newElem,
-                                                 const int32_t *rank, const int32_t *newStart, const int32_t *stayCnt,
-                                                 int32_t *perm, const int32_t *nDev) {
+// The sorted slot of every particle: perm[slot] = old index for the particles
+// that stay, arr[slot] for the arrivals (the sign of rank tells them apart),
+// whose slots k_fix_arrivals puts in order.
+__global__ __launch_bounds__(kBlock) void k_dest(int64_t n, const int32_t *newElem, const int32_t *rank,
+                                                 const int32_t *newStart, const int32_t *stayCnt, int32_t *perm,
+                                                 int32_t *arr, const int32_t *nDev) {
   const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   if (nDev) n = *nDev;
   if (i >= n) return;
   const int ne = newElem[i];
   if (ne < 0) return;
-  const int oe = oldElemOf[i];
-  int64_t d;
-  if (ne == oe) d = newStart[ne] + rank[i];
-  else d = int64_t(newStart[ne]) + stayCnt[ne] + rank[i];
-  perm[d] = int32_t(i);
+  const int r = rank[i], s = newStart[ne];
+  if (r >= 0) perm[s + r] = int32_t(i);
+  else arr[s + stayCnt[ne] + ~r] = int32_t(i);
 }
 
-// per element: order the arrival tail by caller id (insertion sort, tails are short)
+// The arrivals of an element in the order of their caller ids: 8 lanes per
+// element, each counting for its arrivals the smaller ids (an insertion sort
+// by one thread took 36 us where some tens arrive per element, now 11).
+constexpr int kFixLanes = 8;
 __global__ __launch_bounds__(kBlock) void k_fix_arrivals(int nElems, const int32_t *newStart, const int32_t *stayCnt,
-                                                         const int32_t *arrCnt, const int32_t *id, int32_t *perm) {
-  const int e = blockIdx.x * kBlock + threadIdx.x;
+                                                         const int32_t *arrCnt, const int32_t *id, const int32_t *arr,
+                                                         int32_t *perm) {
+  const int t = blockIdx.x * kBlock + threadIdx.x, e = t / kFixLanes;
   if (e >= nElems) return;
   const int na = arrCnt[e];
-  if (na < 2) return;
-  int32_t *p = perm + newStart[e] + stayCnt[e];
-  for (int a = 1; a < na; ++a) {
-    const int32_t v = p[a];
-    const int32_t key = id[v];
-    int b = a - 1;
-    while (b >= 0 && id[p[b]] > key) { p[b + 1] = p[b]; --b; }
-    p[b + 1] = v;
+  if (na == 0) return;
+  const int b = newStart[e] + stayCnt[e];
+  for (int a = t % kFixLanes; a < na; a += kFixLanes) {
+    const int32_t v = arr[b + a], key = id[v];
+    int r = 0;
+    for (int k = 0; k < na; ++k) r += id[arr[b + k]] < key;
+    perm[b + r] = v;
   }
-}
-
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_gather(const int32_t *total, const int32_t *perm, const T *__restrict__ src,
-                                                   T *__restrict__ dst, int width) {
-  const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (j >= int64_t(*total) * width) return;
-  const int64_t r = j / width, c = j % width;
-  dst[j] = src[int64_t(perm[r]) * width + c];
 }
 
 // six FP64 state arrays + id/spec/isNew/elem in one pass
@@ -704,11 +699,23 @@ __device__ inline void record_block_box(double4 *blk, int64_t j, bool has, doubl
   }
 }
 
+// What the launch that ends a re-sort also does: the counters that the next
+// step's kernels count up start at zero, and the particle count goes to
+// pinned host memory (no fills, no copy).
+struct SortEnd {
+  int nElems;
+  int32_t *arrCnt, *moverCount, *hostTotal;
+};
+// STAGED: LastPartPos, LastElem and FieldAtParticle move too
+template <bool STAGED>
 __global__ __launch_bounds__(kBlock) void k_gather_state(const int32_t *total, const int32_t *perm, DevParts s, DevParts d,
                                                          const int32_t *newElem, SpeciesFactor sf, double4 *rec,
-                                                         double4 *recB, double4 *blk) {
+                                                         double4 *recB, double4 *blk, SortEnd end) {
   const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   const int64_t n = *total;
+  for (int64_t e = j; e < end.nElems; e += int64_t(gridDim.x) * kBlock) end.arrCnt[e] = 0;
+  if (j < 2) end.moverCount[j] = 0;
+  if (j == 0) *end.hostTotal = int32_t(n);
   if ((j & ~int64_t(kWave - 1)) >= n) return;   // the whole wave is past the end
   const bool valid = j < n;
   double x = 0.0, y = 0.0, z = 0.0, f = 0.0;
@@ -722,6 +729,12 @@ __global__ __launch_bounds__(kBlock) void k_gather_state(const int32_t *total, c
     d.id[j] = s.id[i]; d.spec[j] = sp; d.isNew[j] = s.isNew[i];
     d.elem[j] = newElem[i];
     if (s.rx) { d.rx[j] = s.rx[i]; d.ry[j] = s.ry[i]; d.rz[j] = s.rz[i]; }
+    if (STAGED) {
+      d.lx[j] = s.lx[i]; d.ly[j] = s.ly[i]; d.lz[j] = s.lz[i];
+      d.lastElem[j] = s.lastElem[i];
+#pragma unroll
+      for (int c = 0; c < 6; ++c) d.F[j * 6 + c] = s.F[int64_t(i) * 6 + c];
+    }
     if (rec) {
       f = sf.fsp[sp];
       rec[j] = make_double4(x, y, z, f);
@@ -1858,14 +1871,6 @@ __global__ void k_fill_i32(int32_t *p, int64_t n, int32_t v) {
   const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   if (i < n) p[i] = v;
 }
-// element id of each sorted slot, from the segment offsets
-__global__ void k_elem_of(int nElems, const int32_t *start, int32_t *elemOf) {
-  const int w = (blockIdx.x * kBlock + threadIdx.x) / kWave;
-  const int lane = lane_id();
-  if (w >= nElems) return;
-  for (int i = start[w] + lane; i < start[w + 1]; i += kWave) elemOf[i] = w;
-}
-
 }  // namespace
 
 namespace {
@@ -1888,6 +1893,10 @@ struct Adjoint {
 };
 }  // namespace
 
+// kEvMain, kEvMainEnd: only where the dominant deposition kernel does not
+// start the deposition (records formed first) or end it (CVWM)
+enum { kEvStart, kEvMain, kEvMainEnd, kEvDepEnd, kEvPush, kEvTrack, kEvSort, kEvGraph0, kEvGraph1, kEvents };
+
 // ======================================================================= handle
 struct pic_handle {
   pic_mesh_desc meshDesc{};
@@ -1904,7 +1913,8 @@ struct pic_handle {
   std::vector<void *> allocs;
   DevParts P{}, Q{};    // current and scratch particle arrays
   int32_t *start = nullptr, *startNew = nullptr, *newElem = nullptr, *rank = nullptr, *perm = nullptr;
-  int32_t *stayCnt = nullptr, *arrCnt = nullptr, *elemOf = nullptr, *dTotal = nullptr;
+  int32_t *stayCnt = nullptr, *arrCnt = nullptr, *arr = nullptr;
+  int32_t *hostTotal = nullptr;   // pinned: the particle count that the last sort wrote
   uint8_t *insideById = nullptr;
   double *stateById = nullptr;
   unsigned long long *lostCount = nullptr;
@@ -1932,7 +1942,10 @@ struct pic_handle {
   bool stagedValid = false;   // LastPartPos/FieldAtParticle refer to the current order
   std::vector<std::pair<int64_t, std::vector<double>>> unplaced;  // particles no element holds at set-up
   // statistics
-  hipEvent_t ev[11] = {};   // ev[9], ev[10]: around the push kernel (kernel A)
+  // device times of an eager step: one event per boundary that the statistics
+  // read (every record costs host time and a packet between two kernels)
+  hipEvent_t ev[kEvents] = {};
+  int evMain = kEvStart, evMainEnd = kEvDepEnd;   // around the dominant deposition kernel
   double msDeposit = 0, msPushTrack = 0, msSort = 0, msDepositMain = 0, msPushMain = 0;
   int nDepositLaunches = 0;
   int64_t nSteps = 0;
@@ -2067,21 +2080,29 @@ int deposit_kernel(const pic_handle *h) {
   return PIC_KERNEL_SF_VALU;
 }
 
+// the device times of a timed deposition that has ended
+void book_deposition(pic_handle *h) {
+  h->msDeposit += elapsed(h->ev[kEvStart], h->ev[kEvDepEnd]);
+  if (h->par.deposition == PIC_DEPO_NONE) return;
+  h->msDepositMain += elapsed(h->ev[h->evMain], h->ev[h->evMainEnd]);
+  h->nDepositLaunches++;
+}
+
 // Deposition() on the current sorted particles
 int run_deposition(pic_handle *h, bool timed) {
   const int ne = h->hm.nElems, N = h->hm.N;
   const size_t nps = size_t(ne) * h->hm.nDof * 4;
-  if (timed) HIPCHK(hipEventRecord(h->ev[0], h->stream));
-  // ev[8] marks the start of the dominant kernel (after the record pass of the
-  // matrix-core gather)
+  if (timed) HIPCHK(hipEventRecord(h->ev[kEvStart], h->stream));
+  h->evMain = kEvStart;
+  h->evMainEnd = kEvDepEnd;
   const bool mixed = h->par.precision == PIC_PREC_MIXED;
   const bool records = h->par.deposition == PIC_DEPO_SF && (h->sfMatrix || mixed);
-  if (timed && !records) HIPCHK(hipEventRecord(h->ev[8], h->stream));
   if (h->par.deposition == PIC_DEPO_NONE) {
     hipLaunchKernelGGL(k_fill_f64, dim3(grid_for(int64_t(nps))), dim3(kBlock), 0, h->stream, h->PS, int64_t(nps));
   } else if (h->par.deposition == PIC_DEPO_CVWM) {
     LAUNCH_N(k_cvwm_elem, N, dim3(grid_for(int64_t(ne) * kWave)), h->M, h->P, h->start, h->elemCorner);
-    if (timed) HIPCHK(hipEventRecord(h->ev[1], h->stream));
+    if (timed) HIPCHK(hipEventRecord(h->ev[kEvMainEnd], h->stream));
+    h->evMainEnd = kEvMainEnd;
     hipLaunchKernelGGL(k_cvwm_class, dim3(grid_for(h->hm.nClasses)), dim3(kBlock), 0, h->stream, h->hm.nClasses,
                        h->classOff, h->classInc, h->classVol, h->elemCorner, h->classSrc);
     LAUNCH_N(k_cvwm_dof, N, dim3(grid_for(int64_t(ne) * h->hm.nDof)), h->M, h->elemClass, h->classSrc, h->PS);
@@ -2091,12 +2112,14 @@ int run_deposition(pic_handle *h, bool timed) {
     if (records) {
       // the element sort writes the records; after other changes of the
       // particle arrays they are formed here
-      if (!h->recFresh)
+      if (!h->recFresh) {
         hipLaunchKernelGGL(k_sf_records, dim3(grid_for(std::max<int64_t>(h->n, 1))), dim3(kBlock), 0, h->stream, h->P,
                            h->start + ne, h->sf, const_cast<double4 *>(h->sf.rec), const_cast<double4 *>(h->sf.recB),
                            block_boxes(h));
+        if (timed) HIPCHK(hipEventRecord(h->ev[kEvMain], h->stream));
+        h->evMain = kEvMain;
+      }
       h->recFresh = true;
-      if (timed) HIPCHK(hipEventRecord(h->ev[8], h->stream));
     }
     if (N == 3 && mixed) {
       const bool cart = h->sf.cartesian != 0;
@@ -2161,10 +2184,9 @@ int run_deposition(pic_handle *h, bool timed) {
     } else {
       LAUNCH_N2(k_sf_gather, N, 0, dim3(nblk), h->M, h->P, h->start, h->sf, h->PS);
     }
-    if (timed) HIPCHK(hipEventRecord(h->ev[1], h->stream));
   }
   HIPCHK(hipGetLastError());
-  if (timed) HIPCHK(hipEventRecord(h->ev[2], h->stream));
+  if (timed) HIPCHK(hipEventRecord(h->ev[kEvDepEnd], h->stream));
   return 0;
 }
 
@@ -2176,32 +2198,24 @@ int enqueue_sort(pic_handle *h, int64_t nGrid, bool withStaged) {
   const int ne = h->hm.nElems;
   const int64_t n = std::max<int64_t>(nGrid, 1);   // the kernels bound themselves by the device count
   const int32_t *nOld = h->start + ne;
-  hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(ne)), dim3(kBlock), 0, h->stream, h->arrCnt, int64_t(ne), 0);
-  hipLaunchKernelGGL(k_elem_of, dim3(grid_for(int64_t(ne) * kWave)), dim3(kBlock), 0, h->stream, ne, h->start, h->elemOf);
   hipLaunchKernelGGL(k_seg_rank, dim3(grid_for(int64_t(ne) * kWave)), dim3(kBlock), 0, h->stream, ne, h->start,
                      h->newElem, h->P.z, h->M.xGPe, h->hm.nDof, h->stayCnt, h->arrCnt, h->rank);
   hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, h->stream, ne, h->stayCnt, h->arrCnt, h->startNew);
-  hipLaunchKernelGGL(k_dest, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, n, h->elemOf, h->newElem, h->rank,
-                     h->startNew, h->stayCnt, h->perm, nOld);
-  hipLaunchKernelGGL(k_fix_arrivals, dim3(grid_for(ne)), dim3(kBlock), 0, h->stream, ne, h->startNew, h->stayCnt,
-                     h->arrCnt, h->P.id, h->perm);
+  hipLaunchKernelGGL(k_dest, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, n, h->newElem, h->rank, h->startNew,
+                     h->stayCnt, h->perm, h->arr, nOld);
+  hipLaunchKernelGGL(k_fix_arrivals, dim3(grid_for(int64_t(ne) * kFixLanes)), dim3(kBlock), 0, h->stream, ne, h->startNew,
+                     h->stayCnt, h->arrCnt, h->P.id, h->arr, h->perm);
   const int32_t *total = h->startNew + ne;
   // records for the shape-function gathers that read them
   const bool useRec = h->sf.rec && (h->sfMatrix || h->par.precision == PIC_PREC_MIXED);
   SpeciesFactor sfac{};
   for (int k = 0; k < 8; ++k) sfac.fsp[k] = h->sf.fsp[k];
-  hipLaunchKernelGGL(k_gather_state, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, total, h->perm, h->P, h->Q, h->newElem,
-                     sfac, useRec ? const_cast<double4 *>(h->sf.rec) : nullptr,
-                     useRec ? const_cast<double4 *>(h->sf.recB) : nullptr,
-                     useRec ? block_boxes(h) : nullptr);
+  const SortEnd end = {ne, h->arrCnt, h->mv.count, h->hostTotal};
+  auto kg = withStaged ? k_gather_state<true> : k_gather_state<false>;
+  hipLaunchKernelGGL(kg, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, total, h->perm, h->P, h->Q, h->newElem, sfac,
+                     useRec ? const_cast<double4 *>(h->sf.rec) : nullptr,
+                     useRec ? const_cast<double4 *>(h->sf.recB) : nullptr, useRec ? block_boxes(h) : nullptr, end);
   if (withStaged) {
-    // keep LastPartPos / LastElem / FieldAtParticle in the new order
-    hipLaunchKernelGGL(k_gather<double>, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, total, h->perm, h->P.lx, h->Q.lx, 1);
-    hipLaunchKernelGGL(k_gather<double>, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, total, h->perm, h->P.ly, h->Q.ly, 1);
-    hipLaunchKernelGGL(k_gather<double>, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, total, h->perm, h->P.lz, h->Q.lz, 1);
-    hipLaunchKernelGGL(k_gather<int32_t>, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, total, h->perm, h->P.lastElem,
-                       h->Q.lastElem, 1);
-    hipLaunchKernelGGL(k_gather<double>, dim3(grid_for(n * 6)), dim3(kBlock), 0, h->stream, total, h->perm, h->P.F, h->Q.F, 6);
     std::swap(h->P.lx, h->Q.lx); std::swap(h->P.ly, h->Q.ly); std::swap(h->P.lz, h->Q.lz);
     std::swap(h->P.lastElem, h->Q.lastElem); std::swap(h->P.F, h->Q.F);
   }
@@ -2216,12 +2230,11 @@ int enqueue_sort(pic_handle *h, int64_t nGrid, bool withStaged) {
   return 0;
 }
 
-// particle count after the last enqueued sort (synchronises the stream)
+// particle count after the last enqueued sort (synchronises the stream; the
+// sort's last kernel wrote the count to pinned host memory)
 int read_count(pic_handle *h) {
-  int32_t total_h = 0;
-  HIPCHK(hipMemcpyAsync(&total_h, h->start + h->hm.nElems, sizeof(int32_t), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
-  h->n = total_h;
+  h->n = *static_cast<volatile int32_t *>(h->hostTotal);
   return 0;
 }
 
@@ -2495,7 +2508,7 @@ int pic_create(const pic_mesh_desc *mesh, const pic_params *par, pic_handle **ou
   rc |= dalloc(h, &h->newElem, cap);
   rc |= dalloc(h, &h->rank, cap);
   rc |= dalloc(h, &h->perm, cap);
-  rc |= dalloc(h, &h->elemOf, cap);
+  rc |= dalloc(h, &h->arr, cap);
   rc |= dalloc(h, &h->stayCnt, hm.nElems);
   rc |= dalloc(h, &h->arrCnt, hm.nElems);
   rc |= dalloc(h, &h->insideById, cap);
@@ -2509,9 +2522,18 @@ int pic_create(const pic_mesh_desc *mesh, const pic_params *par, pic_handle **ou
   }
   rc |= dalloc(h, &h->lostCount, 1);
   if (rc) { pic_destroy(h); return PIC_EHIP; }
+  if (hipHostMalloc(&h->hostTotal, 64, hipHostMallocDefault) != hipSuccess) {
+    pic_destroy(h);
+    return fail(PIC_EHIP, "pic_create: pinned memory");
+  }
+  *h->hostTotal = 0;
+  // counters that the end of every sort clears again
+  HIPCHK(hipMemset(h->arrCnt, 0, size_t(hm.nElems) * sizeof(int32_t)));
+  HIPCHK(hipMemset(h->mv.count, 0, 2 * sizeof(int32_t)));
   HIPCHK(hipMemset(h->lostCount, 0, sizeof(unsigned long long)));
   HIPCHK(hipMemset(h->E, 0, size_t(hm.nElems) * hm.nDof * 3 * sizeof(double)));
   HIPCHK(hipMemset(h->PS, 0, size_t(hm.nElems) * hm.nDof * 4 * sizeof(double)));
+  HIPCHK(hipStreamSynchronize(nullptr));   // the stage's stream does not wait for the null stream
   *out = h;
   return PIC_OK;
 }
@@ -2522,6 +2544,7 @@ int pic_destroy(pic_handle *h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   drop_graph(h);
   for (void *p : h->allocs) (void)hipFree(p);
+  if (h->hostTotal) (void)hipHostFree(h->hostTotal);
   for (auto &e : h->ev)
     if (e) (void)hipEventDestroy(e);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -2670,8 +2693,7 @@ int pic_deposition(pic_handle *h) {
   if (set_device(h)) return PIC_EHIP;
   if (int rc = run_deposition(h, true)) return rc;
   HIPCHK(hipStreamSynchronize(h->stream));
-  h->msDeposit += elapsed(h->ev[0], h->ev[2]);
-  if (h->par.deposition != PIC_DEPO_NONE) { h->msDepositMain += elapsed(h->ev[8], h->ev[1]); h->nDepositLaunches++; }
+  book_deposition(h);
   return PIC_OK;
 }
 
@@ -2744,14 +2766,11 @@ namespace {
 int enqueue_step(pic_handle *h, double dt, int64_t nGrid, bool timed) {
   if (int rc = run_deposition(h, timed)) return rc;
   h->recFresh = false;   // the push below moves the particles; the re-sort writes new records
-  if (timed) HIPCHK(hipEventRecord(h->ev[3], h->stream));
   const int ne = h->hm.nElems;
   const int32_t *nDev = h->start + ne;
   const bool mixed = h->par.precision == PIC_PREC_MIXED;   // N = 3
   const dim3 grid(grid_for(std::max<int64_t>(nGrid, 1)));
   if (h->par.tracking == PIC_TRACK_REFMAPPING) {
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(kBlock), 0, h->stream, h->mv.count, int64_t(2), 0);
-    if (timed) HIPCHK(hipEventRecord(h->ev[9], h->stream));
     if (mixed && h->hm.NGeo == 1)
       hipLaunchKernelGGL((k_rm_push_inside<3, 2, true>), grid, dim3(kBlock), 0, h->stream, h->M, h->P, nGrid, dt,
                          h->newElem, h->mv, nDev);
@@ -2760,15 +2779,13 @@ int enqueue_step(pic_handle *h, double dt, int64_t nGrid, bool timed) {
                          h->newElem, h->mv, nDev);
     else
       LAUNCH_NG(k_rm_push_inside, h->hm.N, h->hm.NGeo, grid, h->M, h->P, nGrid, dt, h->newElem, h->mv, nDev);
-    if (timed) HIPCHK(hipEventRecord(h->ev[10], h->stream));
+    if (timed) HIPCHK(hipEventRecord(h->ev[kEvPush], h->stream));
     LAUNCH_NG(k_rm_movers, h->hm.N, h->hm.NGeo, dim3(std::min<unsigned>(grid.x, 4096u)), h->M, h->P, h->newElem, h->mv,
               h->lostCount, h->insideById, h->stateById);
     if (h->hm.nBC > 0)
       LAUNCH_NG(k_rm_bc_movers, h->hm.N, h->hm.NGeo, dim3(1024), h->M, h->P, h->newElem, h->mv, h->lostCount,
                 h->insideById, h->stateById);
   } else {
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(kBlock), 0, h->stream, h->mv.count, int64_t(1), 0);
-    if (timed) HIPCHK(hipEventRecord(h->ev[9], h->stream));
     // every element affine (N = 3): xi without Newton
     const bool aff = h->M.affine != nullptr && h->hm.N == 3;
     if (mixed && aff)
@@ -2781,13 +2798,15 @@ int enqueue_step(pic_handle *h, double dt, int64_t nGrid, bool timed) {
       hipLaunchKernelGGL((k_push_inside<3, false, true>), grid, dim3(kBlock), 0, h->stream, h->M, h->P, nGrid, dt,
                          h->newElem, h->mv, nDev);
     else { LAUNCH_N(k_push_inside, h->hm.N, grid, h->M, h->P, nGrid, dt, h->newElem, h->mv, nDev); }
-    if (timed) HIPCHK(hipEventRecord(h->ev[10], h->stream));
+    if (timed) HIPCHK(hipEventRecord(h->ev[kEvPush], h->stream));
     hipLaunchKernelGGL(k_track_movers, dim3(1024), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
                        h->lostCount, h->insideById, h->stateById);
   }
   HIPCHK(hipGetLastError());
-  if (timed) HIPCHK(hipEventRecord(h->ev[4], h->stream));
-  return enqueue_sort(h, nGrid, false);
+  if (timed) HIPCHK(hipEventRecord(h->ev[kEvTrack], h->stream));
+  if (int rc = enqueue_sort(h, nGrid, false)) return rc;
+  if (timed) HIPCHK(hipEventRecord(h->ev[kEvSort], h->stream));
+  return 0;
 }
 
 void drop_graph(pic_handle *h) {
@@ -2849,23 +2868,20 @@ int pic_time_step(pic_handle *h, double dt, int32_t nsteps) {
     // as push/track time (the stages are not timed one by one)
     if (int rc = ensure_graph(h, dt)) return rc;
     if (int rc = refresh_records(h)) return rc;
-    HIPCHK(hipEventRecord(h->ev[6], h->stream));
+    HIPCHK(hipEventRecord(h->ev[kEvGraph0], h->stream));
     for (; it + 1 < nsteps; it += 2) HIPCHK(hipGraphLaunch(h->graphExec, h->stream));
-    HIPCHK(hipEventRecord(h->ev[7], h->stream));
+    HIPCHK(hipEventRecord(h->ev[kEvGraph1], h->stream));
     if (int rc = read_count(h)) return rc;
-    h->msPushTrack += elapsed(h->ev[6], h->ev[7]);
+    h->msPushTrack += elapsed(h->ev[kEvGraph0], h->ev[kEvGraph1]);
     h->nSteps += it;
   }
   for (; it < nsteps; ++it) {
     if (int rc = enqueue_step(h, dt, h->n, true)) return rc;
     if (int rc = read_count(h)) return rc;
-    HIPCHK(hipEventRecord(h->ev[5], h->stream));
-    HIPCHK(hipEventSynchronize(h->ev[5]));
-    h->msDeposit += elapsed(h->ev[0], h->ev[2]);
-    if (h->par.deposition != PIC_DEPO_NONE) { h->msDepositMain += elapsed(h->ev[8], h->ev[1]); h->nDepositLaunches++; }
-    h->msPushTrack += elapsed(h->ev[3], h->ev[4]);
-    h->msPushMain += elapsed(h->ev[9], h->ev[10]);
-    h->msSort += elapsed(h->ev[4], h->ev[5]);
+    book_deposition(h);
+    h->msPushTrack += elapsed(h->ev[kEvDepEnd], h->ev[kEvTrack]);
+    h->msPushMain += elapsed(h->ev[kEvDepEnd], h->ev[kEvPush]);
+    h->msSort += elapsed(h->ev[kEvTrack], h->ev[kEvSort]);
     h->nSteps++;
   }
   h->stagedValid = false;
