@@ -659,13 +659,11 @@ int sc_push(pic_handle *h, double dt, const double *E) {
   DevMesh M = h->M;
   M.E = E;
   const dim3 grid(grid_for(std::max<int64_t>(n, 1)));
-  if (M.affine && h->hm.N == 3)   // every element affine: xi without Newton
-    hipLaunchKernelGGL((k_push_inside<3, false, true>), grid, dim3(kBlock), 0, h->stream, M, h->P, n, dt, h->newElem,
-                       h->mv, nDev);
+  if (M.affine) { LAUNCH_N3(k_push_inside, h->hm.N, false, true, grid, M, h->P, n, dt, h->newElem, h->mv, nDev); }
   else
     LAUNCH_N(k_push_inside, h->hm.N, grid, M, h->P, n, dt, h->newElem, h->mv, nDev);
   h->recFresh = false;
-  hipLaunchKernelGGL(k_track_movers, dim3(1024), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
+  hipLaunchKernelGGL(k_track_movers<false>, dim3(1024), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
                      h->lostCount, h->insideById, h->stateById);
   HIPCHK(hipGetLastError());
   return enqueue_sort(h, n, false);
@@ -857,11 +855,9 @@ int pic_adjoint(pic_handle *h, double dt, int32_t K, int32_t every, double *loss
       DevMesh Mstep = h->M;
       Mstep.E = keep ? a.Es[it] : a.seg[it - s0].E;
       if (S.n > 0) {
-        if (Mstep.affine && N == 3)
-          hipLaunchKernelGGL((k_adj_push<3, true>), dim3(grid_for(S.n)), dim3(kBlock), 0, h->stream, Mstep, V, S.n, dt,
-                             a.lx, a.lv, a.lF, a.xi);
-        else
-          LAUNCH_N2(k_adj_push, N, false, dim3(grid_for(S.n)), Mstep, V, S.n, dt, a.lx, a.lv, a.lF, a.xi);
+        const dim3 grid(grid_for(S.n));
+        if (Mstep.affine) { LAUNCH_N2(k_adj_push, N, true, grid, Mstep, V, S.n, dt, a.lx, a.lv, a.lF, a.xi); }
+        else { LAUNCH_N2(k_adj_push, N, false, grid, Mstep, V, S.n, dt, a.lx, a.lv, a.lF, a.xi); }
       }
       LAUNCH_N(k_adj_scatter, N, dim3(ne), Mstep, S.start, a.lF, a.xi, a.lE);
       HIPCHK(hipGetLastError());

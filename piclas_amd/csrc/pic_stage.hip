@@ -68,13 +68,16 @@ __device__ inline int lane_id() { return __lane_id(); }
 template <int N, bool MIXED = false, bool AFFINE = false>
 __global__ __launch_bounds__(kBlock) void k_interp(DevMesh M, DevParts P, int64_t n) {
   const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  const int e = i < n ? P.elem[i] : -1;
+  const int eu = __builtin_amdgcn_readfirstlane(e);
+  const bool uni = eu >= 0 && __ballot(i < n && e != eu) == 0;   // as in k_push_inside
   if (i >= n) return;
-  const int e = P.elem[i];
   double F[6] = {0, 0, 0, 0, 0, 0};
   const int sp = P.spec[i];
   if (e >= 0 && fabs(M.charge[sp]) > 0.0) {
     const double x[3] = {P.x[i], P.y[i], P.z[i]};
-    field_at_particle<N, MIXED, AFFINE>(M, e, x, F);
+    if (uni) field_at_particle<N, MIXED, AFFINE, true>(M, eu, x, F);
+    else field_at_particle<N, MIXED, AFFINE>(M, e, x, F);
   }
 #pragma unroll
   for (int c = 0; c < 6; ++c) P.F[i * 6 + c] = F[c];
@@ -100,64 +103,6 @@ __global__ __launch_bounds__(kBlock) void k_push(DevMesh M, DevParts P, int64_t 
   P.vx[i] = v[0]; P.vy[i] = v[1]; P.vz[i] = v[2];
 }
 
-// Tracking only (PerformTracking): from lastElem / LastPartPos to the new owner
-__global__ __launch_bounds__(kBlock) void k_track(DevMesh M, DevParts P, int64_t n, int32_t *newElem,
-                                                  unsigned long long *lostCount, uint8_t *insideById, double *stateById) {
-  const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int e0 = P.lastElem[i];
-  if (e0 < 0) { newElem[i] = -1; return; }
-  double x[3] = {P.x[i], P.y[i], P.z[i]};
-  double last[3] = {P.lx[i], P.ly[i], P.lz[i]};
-  bool lost;
-  int steps;
-  const int e = tria_track(M, e0, x, last, lost, steps);
-  P.x[i] = x[0]; P.y[i] = x[1]; P.z[i] = x[2];
-  P.lx[i] = last[0]; P.ly[i] = last[1]; P.lz[i] = last[2];
-  newElem[i] = e;
-  P.elem[i] = e;
-  if (e < 0) {
-    const int id = P.id[i];
-    insideById[id] = 0;
-    double *st = stateById + (size_t)id * 6;
-    st[0] = x[0]; st[1] = x[1]; st[2] = x[2]; st[3] = P.vx[i]; st[4] = P.vy[i]; st[5] = P.vz[i];
-    if (lost) atomicAdd(lostCount, 1ull);
-  }
-}
-
-// Fused step body: interpolate + push + track for one particle
-template <int N>
-__global__ __launch_bounds__(kBlock) void k_push_track(DevMesh M, DevParts P, int64_t n, double dt, int32_t *newElem,
-                                                       unsigned long long *lostCount, uint8_t *insideById,
-                                                       double *stateById) {
-  const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int e0 = P.elem[i];
-  if (e0 < 0) { newElem[i] = -1; return; }
-  double x[3] = {P.x[i], P.y[i], P.z[i]};
-  double v[3] = {P.vx[i], P.vy[i], P.vz[i]};
-  const double last0[3] = {x[0], x[1], x[2]};
-  const int sp = P.spec[i];
-  double F[6] = {0, 0, 0, 0, 0, 0};
-  if (fabs(M.charge[sp]) > 0.0) field_at_particle<N>(M, e0, x, F);
-  boris_push(M.charge[sp], M.mass[sp], P.isNew[i] != 0, F, dt, x, v);
-  double last[3] = {last0[0], last0[1], last0[2]};
-  bool lost;
-  int steps;
-  const int e = tria_track(M, e0, x, last, lost, steps);
-  P.x[i] = x[0]; P.y[i] = x[1]; P.z[i] = x[2];
-  P.vx[i] = v[0]; P.vy[i] = v[1]; P.vz[i] = v[2];
-  P.isNew[i] = 0;
-  newElem[i] = e;
-  if (e < 0) {
-    const int id = P.id[i];
-    insideById[id] = 0;
-    double *st = stateById + (size_t)id * 6;
-    st[0] = x[0]; st[1] = x[1]; st[2] = x[2]; st[3] = v[0]; st[4] = v[1]; st[5] = v[2];
-    if (lost) atomicAdd(lostCount, 1ull);
-  }
-}
-
 // Split form of the fused step for throughput.  Kernel A does, per particle,
 // interpolate + push and the first iteration of SingleParticleTriaTracking3D
 // (ParticleInsideQuad3D in the last element); particles still inside are
@@ -172,6 +117,38 @@ struct Movers {
   uint8_t *flag;    // [cap] RefMapping: bit 0 boundary candidate, bit 1 still inside its element
   int32_t *slot2;   // [cap] RefMapping: the slots that k_rm_bc_filter passes on (count at count[1])
 };
+
+// one atomic per wave for the slots of the lanes that are movers
+__device__ inline int mover_slot(int32_t *count, bool mover) {
+  const unsigned long long m = __ballot(mover);
+  if (m == 0) return 0;
+  const int lane = lane_id();
+  const int leader = __ffsll((long long)m) - 1;
+  int base = 0;
+  if (lane == leader) base = atomicAdd(count, __popcll(m));
+  base = __shfl(base, leader, kWave);
+  return base + __popcll(m & ((1ull << lane) - 1ull));
+}
+
+// The first iteration of SingleParticleTriaTracking3D: whether x is inside
+// element e.  On a parallelepiped (AFFINE: corner map affine to 1e-14)
+// ParticleInsideQuad3D decides as |xi| <= 1 does, xi = A^-1 (x - c), except
+// within rounding of a face: the reference's side test runs only for
+// particles with max |xi| within 1e-10 of 1, the others are decided by xi.
+// (uni: e is wave-uniform)
+template <bool AFFINE>
+__device__ inline bool inside_elem(const DevMesh &M, int e, bool uni, const double x[3]) {
+  double det[6][2];
+  if (AFFINE) {
+    double xi[3];
+    if (uni) affine_xi<true>(M, e, x, xi);
+    else affine_xi(M, e, x, xi);
+    const double mx = max_abs3(xi);
+    if (mx < 1.0 - 1e-10) return true;
+    if (mx > 1.0 + 1e-10) return false;
+  }
+  return uni ? inside_quad<true>(M, e, x, det) : inside_quad(M, e, x, det);
+}
 
 template <int N, bool MIXED = false, bool AFFINE = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_PUSH))) void k_push_inside(DevMesh M, DevParts P, int64_t n, double dt, int32_t *newElem,
@@ -203,37 +180,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_PUSH
       P.x[i] = x[0]; P.y[i] = x[1]; P.z[i] = x[2];
       P.vx[i] = v[0]; P.vy[i] = v[1]; P.vz[i] = v[2];
       P.isNew[i] = 0;
-      double det[6][2];
-      bool in;
-      if (AFFINE) {
-        // On a parallelepiped (corner map affine to 1e-14) ParticleInsideQuad3D
-        // decides as |xi| <= 1 does, xi = A^-1 (x - c), except within rounding
-        // of a face: the reference's side test runs only for particles with
-        // max |xi| within 1e-10 of 1, the others are decided by xi.
-        double xi[3];
-        if (uni) affine_xi<true>(M, eu, x, xi);
-        else affine_xi(M, e0, x, xi);
-        const double mx = max_abs3(xi);
-        if (mx < 1.0 - 1e-10) in = true;
-        else if (mx > 1.0 + 1e-10) in = false;
-        else in = uni ? inside_quad<true>(M, eu, x, det) : inside_quad(M, e0, x, det);
-      } else {
-        in = uni ? inside_quad<true>(M, eu, x, det) : inside_quad(M, e0, x, det);
-      }
-      if (in) newElem[i] = e0;
+      if (inside_elem<AFFINE>(M, uni ? eu : e0, uni, x)) newElem[i] = e0;
       else mover = true;
     }
   }
-  // one atomic per wave for the mover slots
-  const unsigned long long m = __ballot(mover);
-  if (m == 0) return;
-  const int lane = lane_id();
-  const int leader = __ffsll((long long)m) - 1;
-  int base = 0;
-  if (lane == leader) base = atomicAdd(mv.count, __popcll(m));
-  base = __shfl(base, leader, kWave);
+  const int slot = mover_slot(mv.count, mover);
   if (mover) {
-    const int slot = base + __popcll(m & ((1ull << lane) - 1ull));
     mv.idx[slot] = int32_t(i);
     mv.last[(size_t)slot * 3 + 0] = last[0];
     mv.last[(size_t)slot * 3 + 1] = last[1];
@@ -241,6 +193,36 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_PUSH
   }
 }
 
+// Staged PerformTracking, in the same split: the particles still inside
+// LastElem are done (their LastPartPos stays), the others go to the list
+template <bool AFFINE>
+__global__ __launch_bounds__(kBlock) void k_track_inside(DevMesh M, DevParts P, int64_t n, int32_t *newElem, Movers mv) {
+  const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  const int e = i < n ? P.lastElem[i] : -1;
+  const int eu = __builtin_amdgcn_readfirstlane(e);
+  const bool uni = eu >= 0 && __ballot(i < n && e != eu) == 0;
+  bool mover = false;
+  if (i < n) {
+    if (e < 0) {
+      newElem[i] = -1;
+    } else {
+      const double x[3] = {P.x[i], P.y[i], P.z[i]};
+      if (inside_elem<AFFINE>(M, uni ? eu : e, uni, x)) newElem[i] = e;
+      else mover = true;
+    }
+  }
+  const int slot = mover_slot(mv.count, mover);
+  if (mover) {
+    mv.idx[slot] = int32_t(i);
+    mv.last[(size_t)slot * 3 + 0] = P.lx[i];
+    mv.last[(size_t)slot * 3 + 1] = P.ly[i];
+    mv.last[(size_t)slot * 3 + 2] = P.lz[i];
+  }
+}
+
+// The full face walk of the movers.  STAGED: from LastElem, and LastPartPos
+// (shifted across periodic sides) is kept
+template <bool STAGED>
 __global__ __launch_bounds__(kBlock) void k_track_movers(DevMesh M, DevParts P, int32_t *newElem, Movers mv,
                                                          unsigned long long *lostCount, uint8_t *insideById,
                                                          double *stateById) {
@@ -251,8 +233,9 @@ __global__ __launch_bounds__(kBlock) void k_track_movers(DevMesh M, DevParts P, 
     double last[3] = {mv.last[(size_t)k * 3], mv.last[(size_t)k * 3 + 1], mv.last[(size_t)k * 3 + 2]};
     bool lost;
     int steps;
-    const int e = tria_track(M, P.elem[i], x, last, lost, steps);
+    const int e = tria_track(M, STAGED ? P.lastElem[i] : P.elem[i], x, last, lost, steps);
     P.x[i] = x[0]; P.y[i] = x[1]; P.z[i] = x[2];
+    if (STAGED) { P.lx[i] = last[0]; P.ly[i] = last[1]; P.lz[i] = last[2]; }
     newElem[i] = e;
     if (e < 0) {
       const int id = P.id[i];
@@ -334,15 +317,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_RM))
       }
     }
   }
-  const unsigned long long m = __ballot(mover);
-  if (m == 0) return;
-  const int lane = lane_id();
-  const int leader = __ffsll((long long)m) - 1;
-  int base = 0;
-  if (lane == leader) base = atomicAdd(mv.count, __popcll(m));
-  base = __shfl(base, leader, kWave);
+  const int slot = mover_slot(mv.count, mover);
   if (mover) {
-    const int slot = base + __popcll(m & ((1ull << lane) - 1ull));
     mv.idx[slot] = int32_t(i);
     mv.flag[slot] = uint8_t((head.cand ? 1 : 0) | (head.inside ? 2 : 0));
     // LastPartPos: the position before the push, read back from the arrays
@@ -2031,6 +2007,18 @@ int alloc_parts(pic_handle *h, DevParts &P, int64_t cap) {
     default: break;                                                                                 \
   }
 
+#define LAUNCH_N3(KERNEL, N, A2, A3, GRID, ...)                                                        \
+  switch (N) {                                                                                      \
+    case 1: hipLaunchKernelGGL((KERNEL<1, A2, A3>), GRID, dim3(kBlock), 0, h->stream, __VA_ARGS__); break; \
+    case 2: hipLaunchKernelGGL((KERNEL<2, A2, A3>), GRID, dim3(kBlock), 0, h->stream, __VA_ARGS__); break; \
+    case 3: hipLaunchKernelGGL((KERNEL<3, A2, A3>), GRID, dim3(kBlock), 0, h->stream, __VA_ARGS__); break; \
+    case 4: hipLaunchKernelGGL((KERNEL<4, A2, A3>), GRID, dim3(kBlock), 0, h->stream, __VA_ARGS__); break; \
+    case 5: hipLaunchKernelGGL((KERNEL<5, A2, A3>), GRID, dim3(kBlock), 0, h->stream, __VA_ARGS__); break; \
+    case 6: hipLaunchKernelGGL((KERNEL<6, A2, A3>), GRID, dim3(kBlock), 0, h->stream, __VA_ARGS__); break; \
+    case 7: hipLaunchKernelGGL((KERNEL<7, A2, A3>), GRID, dim3(kBlock), 0, h->stream, __VA_ARGS__); break; \
+    default: break;                                                                                 \
+  }
+
 #define LAUNCH_NG_N(KERNEL, N, G, GRID, ...)                                                                  \
   switch (N) {                                                                                                 \
     case 1: hipLaunchKernelGGL((KERNEL<1, G>), GRID, dim3(kBlock), 0, h->stream, __VA_ARGS__); break;           \
@@ -2717,13 +2705,12 @@ int pic_interpolate_field_to_particle(pic_handle *h) {
       if (mixed) hipLaunchKernelGGL((k_rm_interp<3, true>), dim3(grid_for(h->n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->n);
       else { LAUNCH_N(k_rm_interp, h->hm.N, dim3(grid_for(h->n)), h->M, h->P, h->n); }
     } else {
-      const bool aff = h->M.affine != nullptr && h->hm.N == 3;
+      const bool aff = h->M.affine != nullptr;
       if (mixed && aff)
         hipLaunchKernelGGL((k_interp<3, true, true>), dim3(grid_for(h->n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->n);
       else if (mixed)
         hipLaunchKernelGGL((k_interp<3, true>), dim3(grid_for(h->n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->n);
-      else if (aff)
-        hipLaunchKernelGGL((k_interp<3, false, true>), dim3(grid_for(h->n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->n);
+      else if (aff) { LAUNCH_N3(k_interp, h->hm.N, false, true, dim3(grid_for(h->n)), h->M, h->P, h->n); }
       else { LAUNCH_N(k_interp, h->hm.N, dim3(grid_for(h->n)), h->M, h->P, h->n); }
     }
   }
@@ -2755,7 +2742,9 @@ int pic_perform_tracking(pic_handle *h) {
       LAUNCH_NG(k_rm_track, h->hm.N, h->hm.NGeo, dim3(grid_for(h->n)), h->M, h->P, h->n, h->newElem, h->lostCount,
                 h->insideById, h->stateById);
     } else {
-      hipLaunchKernelGGL(k_track, dim3(grid_for(h->n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->n, h->newElem,
+      auto kt = h->M.affine ? k_track_inside<true> : k_track_inside<false>;
+      hipLaunchKernelGGL(kt, dim3(grid_for(h->n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->n, h->newElem, h->mv);
+      hipLaunchKernelGGL(k_track_movers<true>, dim3(1024), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
                          h->lostCount, h->insideById, h->stateById);
     }
     HIPCHK(hipGetLastError());
@@ -2796,20 +2785,17 @@ int enqueue_step(pic_handle *h, double dt, int64_t nGrid, bool timed) {
       LAUNCH_NG(k_rm_bc_movers, h->hm.N, h->hm.NGeo, dim3(1024), h->M, h->P, h->newElem, h->mv, h->lostCount,
                 h->insideById, h->stateById);
   } else {
-    // every element affine (N = 3): xi without Newton
-    const bool aff = h->M.affine != nullptr && h->hm.N == 3;
+    const bool aff = h->M.affine != nullptr;   // every element affine: xi without Newton
     if (mixed && aff)
       hipLaunchKernelGGL((k_push_inside<3, true, true>), grid, dim3(kBlock), 0, h->stream, h->M, h->P, nGrid, dt,
                          h->newElem, h->mv, nDev);
     else if (mixed)
       hipLaunchKernelGGL((k_push_inside<3, true>), grid, dim3(kBlock), 0, h->stream, h->M, h->P, nGrid, dt, h->newElem,
                          h->mv, nDev);
-    else if (aff)
-      hipLaunchKernelGGL((k_push_inside<3, false, true>), grid, dim3(kBlock), 0, h->stream, h->M, h->P, nGrid, dt,
-                         h->newElem, h->mv, nDev);
+    else if (aff) { LAUNCH_N3(k_push_inside, h->hm.N, false, true, grid, h->M, h->P, nGrid, dt, h->newElem, h->mv, nDev); }
     else { LAUNCH_N(k_push_inside, h->hm.N, grid, h->M, h->P, nGrid, dt, h->newElem, h->mv, nDev); }
     if (timed) HIPCHK(hipEventRecord(h->ev[kEvPush], h->stream));
-    hipLaunchKernelGGL(k_track_movers, dim3(1024), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
+    hipLaunchKernelGGL(k_track_movers<false>, dim3(1024), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
                        h->lostCount, h->insideById, h->stateById);
   }
   HIPCHK(hipGetLastError());
