@@ -663,8 +663,8 @@ int sc_push(pic_handle *h, double dt, const double *E) {
   else
     LAUNCH_N(k_push_inside, h->hm.N, grid, M, h->P, n, dt, h->newElem, h->mv, nDev);
   h->recFresh = false;
-  hipLaunchKernelGGL(k_track_movers<false>, dim3(1024), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
-                     h->lostCount, h->insideById, h->stateById);
+  hipLaunchKernelGGL(k_track_movers<false>, dim3(mover_grid(n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem,
+                     h->mv, h->lostCount, h->insideById, h->stateById);
   HIPCHK(hipGetLastError());
   return enqueue_sort(h, n, false);
 }

@@ -106,17 +106,32 @@ __global__ __launch_bounds__(kBlock) void k_push(DevMesh M, DevParts P, int64_t 
 // Split form of the fused step for throughput.  Kernel A does, per particle,
 // interpolate + push and the first iteration of SingleParticleTriaTracking3D
 // (ParticleInsideQuad3D in the last element); particles still inside are
-// done.  The others (about one in a hundred) are appended to a list and
-// kernel B runs the full face walk for them from the same state, so the
-// result is the one of the single loop.  Splitting keeps kernel A's register
-// footprint low enough for several waves per SIMD.
+// done.  The others (about one in a hundred) are appended to a list, their
+// LastPartPos is kept in lx, ly, lz, and kernel B runs the full face walk for
+// them from the same state, so the result is the one of the single loop.
+// Splitting keeps kernel A's register footprint low enough for several waves
+// per SIMD.
+//
+// The list has kMoverSegs segments with a counter each, a cache line apart;
+// a workgroup appends to the one of its index.  With one counter the atomics
+// of the waves queue up at its address: of kernel A's 1557 us (22 million
+// particles, 0.5 % movers) that was 250, of the staged test's 83 us (2 million)
+// 68.  Kernel B finding marks in newElem by itself needs no atomics, but its
+// workgroups hold few movers each (134-238 us for 95).
+constexpr int kMoverSegs = 64, kMoverLine = 16;
+constexpr int kMoverCounters = (kMoverSegs + 1) * kMoverLine;
 struct Movers {
-  int32_t *count;   // [1]
-  int32_t *idx;     // [cap]
-  double *last;     // [cap][3] LastPartPos
-  uint8_t *flag;    // [cap] RefMapping: bit 0 boundary candidate, bit 1 still inside its element
-  int32_t *slot2;   // [cap] RefMapping: the slots that k_rm_bc_filter passes on (count at count[1])
+  int32_t *count;   // [kMoverCounters]: of segment s at s * kMoverLine; of late at kMoverSegs * kMoverLine
+  int32_t *idx;     // [kMoverSegs][seg] particles
+  int64_t seg;      // places per segment
+  int32_t *late;    // [cap] RefMapping: the particles that k_rm_movers passes on
+  double *last;     // [cap][3] positions of particles to be located (set-up)
 };
+// places per segment: all particles of the workgroups that share it
+inline int64_t mover_seg(int64_t cap) { return ((cap + kBlock - 1) / kBlock + kMoverSegs - 1) / kMoverSegs * kBlock; }
+
+// workgroups of kernel B (a multiple of kMoverSegs), of which few find no mover
+inline unsigned mover_grid(int64_t n) { return n < (int64_t(1) << 20) ? 4 * kMoverSegs : 64 * kMoverSegs; }
 
 // one atomic per wave for the slots of the lanes that are movers
 __device__ inline int mover_slot(int32_t *count, bool mover) {
@@ -128,6 +143,13 @@ __device__ inline int mover_slot(int32_t *count, bool mover) {
   if (lane == leader) base = atomicAdd(count, __popcll(m));
   base = __shfl(base, leader, kWave);
   return base + __popcll(m & ((1ull << lane) - 1ull));
+}
+
+// appends the mover lanes' particles to the workgroup's segment
+__device__ inline void add_mover(const Movers &mv, bool mover, int64_t i) {
+  const int s = blockIdx.x % kMoverSegs;
+  const int slot = mover_slot(mv.count + s * kMoverLine, mover);
+  if (mover) mv.idx[s * mv.seg + slot] = int32_t(i);
 }
 
 // The first iteration of SingleParticleTriaTracking3D: whether x is inside
@@ -154,9 +176,8 @@ template <int N, bool MIXED = false, bool AFFINE = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_PUSH))) void k_push_inside(DevMesh M, DevParts P, int64_t n, double dt, int32_t *newElem,
                                                         Movers mv, const int32_t *nDev) {
   const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (nDev) n = *nDev;   // particle count on the device (graph replay)
-  bool mover = false;
-  double last[3] = {0, 0, 0};
+  if (nDev) n = *nDev;
+  bool mover = false;   // particle count on the device (graph replay)
   // whether all particles of the wave sit in one element (sorted order: most
   // waves); its field is then read by scalar loads
   const int eAll = i < n ? P.elem[i] : -1;
@@ -169,7 +190,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_PUSH
     } else {
       double x[3] = {P.x[i], P.y[i], P.z[i]};
       double v[3] = {P.vx[i], P.vy[i], P.vz[i]};
-      last[0] = x[0]; last[1] = x[1]; last[2] = x[2];
+      const double last[3] = {x[0], x[1], x[2]};
       const int sp = P.spec[i];
       double F[6] = {0, 0, 0, 0, 0, 0};
       if (fabs(M.charge[sp]) > 0.0) {
@@ -180,17 +201,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_PUSH
       P.x[i] = x[0]; P.y[i] = x[1]; P.z[i] = x[2];
       P.vx[i] = v[0]; P.vy[i] = v[1]; P.vz[i] = v[2];
       P.isNew[i] = 0;
-      if (inside_elem<AFFINE>(M, uni ? eu : e0, uni, x)) newElem[i] = e0;
-      else mover = true;
+      if (inside_elem<AFFINE>(M, uni ? eu : e0, uni, x)) {
+        newElem[i] = e0;
+      } else {
+        mover = true;
+        P.lx[i] = last[0]; P.ly[i] = last[1]; P.lz[i] = last[2];
+      }
     }
   }
-  const int slot = mover_slot(mv.count, mover);
-  if (mover) {
-    mv.idx[slot] = int32_t(i);
-    mv.last[(size_t)slot * 3 + 0] = last[0];
-    mv.last[(size_t)slot * 3 + 1] = last[1];
-    mv.last[(size_t)slot * 3 + 2] = last[2];
-  }
+  add_mover(mv, mover, i);
 }
 
 // Staged PerformTracking, in the same split: the particles still inside
@@ -211,26 +230,23 @@ __global__ __launch_bounds__(kBlock) void k_track_inside(DevMesh M, DevParts P, 
       else mover = true;
     }
   }
-  const int slot = mover_slot(mv.count, mover);
-  if (mover) {
-    mv.idx[slot] = int32_t(i);
-    mv.last[(size_t)slot * 3 + 0] = P.lx[i];
-    mv.last[(size_t)slot * 3 + 1] = P.ly[i];
-    mv.last[(size_t)slot * 3 + 2] = P.lz[i];
-  }
+  add_mover(mv, mover, i);
 }
 
-// The full face walk of the movers.  STAGED: from LastElem, and LastPartPos
-// (shifted across periodic sides) is kept
+// The full face walk of the movers, the grid a multiple of kMoverSegs
+// workgroups.  STAGED: from LastElem, and LastPartPos (shifted across
+// periodic sides) is kept
 template <bool STAGED>
 __global__ __launch_bounds__(kBlock) void k_track_movers(DevMesh M, DevParts P, int32_t *newElem, Movers mv,
                                                          unsigned long long *lostCount, uint8_t *insideById,
                                                          double *stateById) {
-  const int cnt = *mv.count;
-  for (int k = blockIdx.x * kBlock + threadIdx.x; k < cnt; k += gridDim.x * kBlock) {
-    const int i = mv.idx[k];
+  const int s = blockIdx.x % kMoverSegs;
+  const int cnt = mv.count[s * kMoverLine];
+  const int32_t *idx = mv.idx + s * mv.seg;
+  for (int k = blockIdx.x / kMoverSegs * kBlock + threadIdx.x; k < cnt; k += gridDim.x / kMoverSegs * kBlock) {
+    const int i = idx[k];
     double x[3] = {P.x[i], P.y[i], P.z[i]};
-    double last[3] = {mv.last[(size_t)k * 3], mv.last[(size_t)k * 3 + 1], mv.last[(size_t)k * 3 + 2]};
+    double last[3] = {P.lx[i], P.ly[i], P.lz[i]};
     bool lost;
     int steps;
     const int e = tria_track(M, STAGED ? P.lastElem[i] : P.elem[i], x, last, lost, steps);
@@ -287,14 +303,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_RM))
   const int eAll = i < n ? P.elem[i] : -1;
   const int eu = __builtin_amdgcn_readfirstlane(eAll);
   const bool uni = eu >= 0 && __ballot(i < n && eAll != eu) == 0;
-  RmHead head = {true, false};
-  double x[3] = {0, 0, 0};
   if (i < n) {
     const int e0 = eAll;
     if (e0 < 0) {
       newElem[i] = -1;
     } else {
-      x[0] = P.x[i]; x[1] = P.y[i]; x[2] = P.z[i];
+      double x[3] = {P.x[i], P.y[i], P.z[i]};
       double v[3] = {P.vx[i], P.vy[i], P.vz[i]};
       double last[3] = {x[0], x[1], x[2]};
       double xi[3] = {P.rx[i], P.ry[i], P.rz[i]};
@@ -307,29 +321,23 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_RM))
       boris_push(M.charge[sp], M.mass[sp], P.isNew[i] != 0, F, dt, x, v);
       P.vx[i] = v[0]; P.vy[i] = v[1]; P.vz[i] = v[2];
       P.isNew[i] = 0;
-      head = uni ? rm_track_head<N, G, true>(M, eu, x, last, xi) : rm_track_head<N, G>(M, e0, x, last, xi);
+      const RmHead head = uni ? rm_track_head<N, G, true>(M, eu, x, last, xi) : rm_track_head<N, G>(M, e0, x, last, xi);
       P.rx[i] = xi[0]; P.ry[i] = xi[1]; P.rz[i] = xi[2];
       if (head.inside && !head.cand) {
         newElem[i] = e0;
-        P.x[i] = x[0]; P.y[i] = x[1]; P.z[i] = x[2];
       } else {
-        mover = true;   // x is stored after LastPartPos is read back below
+        mover = true;
+        newElem[i] = (head.cand ? 1 : 0) | (head.inside ? 2 : 0);   // for k_rm_movers
+        // LastPartPos: the position before the push, read back from the arrays
+        // (not held in registers across the Newton iteration; after a
+        // PeriodicMovement it is not the shifted one, which no later stage reads
+        // on CartesianPeriodic meshes)
+        P.lx[i] = P.x[i]; P.ly[i] = P.y[i]; P.lz[i] = P.z[i];
       }
+      P.x[i] = x[0]; P.y[i] = x[1]; P.z[i] = x[2];
     }
   }
-  const int slot = mover_slot(mv.count, mover);
-  if (mover) {
-    mv.idx[slot] = int32_t(i);
-    mv.flag[slot] = uint8_t((head.cand ? 1 : 0) | (head.inside ? 2 : 0));
-    // LastPartPos: the position before the push, read back from the arrays
-    // (not held in registers across the Newton iteration; after a
-    // PeriodicMovement it is not the shifted one, which no later stage reads
-    // on CartesianPeriodic meshes)
-    mv.last[(size_t)slot * 3 + 0] = P.x[i];
-    mv.last[(size_t)slot * 3 + 1] = P.y[i];
-    mv.last[(size_t)slot * 3 + 2] = P.z[i];
-    P.x[i] = x[0]; P.y[i] = x[1]; P.z[i] = x[2];
-  }
+  add_mover(mv, mover, i);
 }
 
 // Kernel B for RefMapping: the particles that left their element, and those
@@ -344,19 +352,22 @@ template <int N, int G>
 __global__ __launch_bounds__(kBlock) void k_rm_movers(DevMesh M, DevParts P, int32_t *newElem, Movers mv,
                                                       unsigned long long *lostCount, uint8_t *insideById,
                                                       double *stateById) {
-  const int cnt = *mv.count;
+  const int s = blockIdx.x % kMoverSegs;
+  const int cnt = mv.count[s * kMoverLine];
+  const int32_t *idx = mv.idx + s * mv.seg;
   const int lane = lane_id();
-  const int stride = gridDim.x * kBlock;
   // wave-uniform trip count: every lane takes part in the ballots
-  for (int k0 = blockIdx.x * kBlock + (threadIdx.x & ~(kWave - 1)); k0 < cnt; k0 += stride) {
+  for (int k0 = blockIdx.x / kMoverSegs * kBlock + (threadIdx.x & ~(kWave - 1)); k0 < cnt;
+       k0 += gridDim.x / kMoverSegs * kBlock) {
     const int k = k0 + lane;
     bool defer = false;
+    int i = 0;
     if (k < cnt) {
-      const int i = mv.idx[k];
-      uint8_t f = mv.flag[k];
+      i = idx[k];
+      const int f = newElem[i];   // bit 0 boundary candidate, bit 1 still inside its element
       const int e0 = P.elem[i];
       double x[3] = {P.x[i], P.y[i], P.z[i]};
-      double last[3] = {mv.last[(size_t)k * 3], mv.last[(size_t)k * 3 + 1], mv.last[(size_t)k * 3 + 2]};
+      double last[3] = {P.lx[i], P.ly[i], P.lz[i]};
       bool done = false;
       if (f & 1) {
         const double d0 = x[0] - last[0], d1 = x[1] - last[1], d2 = x[2] - last[2];
@@ -366,8 +377,7 @@ __global__ __launch_bounds__(kBlock) void k_rm_movers(DevMesh M, DevParts P, int
           newElem[i] = e0;
           done = true;
         } else {
-          f = uint8_t(f & ~1);
-          mv.flag[k] = f;
+          newElem[i] = 0;   // (no candidate any more, for the fallback of the search)
         }
       } else if (f & 2) {   // (not a mover: kept for completeness)
         newElem[i] = e0;
@@ -389,13 +399,8 @@ __global__ __launch_bounds__(kBlock) void k_rm_movers(DevMesh M, DevParts P, int
         }
       }
     }
-    const unsigned long long m = __ballot(defer);
-    if (m == 0) continue;
-    const int leader = __ffsll((long long)m) - 1;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(mv.count + 1, __popcll(m));
-    base = __shfl(base, leader, kWave);
-    if (defer) mv.slot2[base + __popcll(m & ((1ull << lane) - 1ull))] = k;
+    const int slot = mover_slot(mv.count + kMoverSegs * kMoverLine, defer);
+    if (defer) mv.late[slot] = i;
   }
 }
 
@@ -406,13 +411,12 @@ template <int N, int G>
 __global__ __launch_bounds__(kBlock) void k_rm_bc_movers(DevMesh M, DevParts P, int32_t *newElem, Movers mv,
                                                          unsigned long long *lostCount, uint8_t *insideById,
                                                          double *stateById) {
-  const int cnt = mv.count[1];
+  const int cnt = mv.count[kMoverSegs * kMoverLine];
   for (int j = blockIdx.x * kBlock + threadIdx.x; j < cnt; j += gridDim.x * kBlock) {
-    const int k = mv.slot2[j];
-    const int i = mv.idx[k];
-    const uint8_t f = mv.flag[k];
+    const int i = mv.late[j];
+    const int f = newElem[i];
     double x[3] = {P.x[i], P.y[i], P.z[i]};
-    double last[3] = {mv.last[(size_t)k * 3], mv.last[(size_t)k * 3 + 1], mv.last[(size_t)k * 3 + 2]};
+    double last[3] = {P.lx[i], P.ly[i], P.lz[i]};
     double xi[3] = {P.rx[i], P.ry[i], P.rz[i]};
     int status;
     const RmHead h = {(f & 2) != 0, (f & 1) != 0};
@@ -690,7 +694,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_state(const int32_t *total, c
   const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   const int64_t n = *total;
   for (int64_t e = j; e < end.nElems; e += int64_t(gridDim.x) * kBlock) end.arrCnt[e] = 0;
-  if (j < 2) end.moverCount[j] = 0;
+  for (int64_t e = j; e < kMoverCounters; e += int64_t(gridDim.x) * kBlock) end.moverCount[e] = 0;
   if (j == 0) *end.hostTotal = int32_t(n);
   if ((j & ~int64_t(kWave - 1)) >= n) return;   // the whole wave is past the end
   const bool valid = j < n;
@@ -2511,12 +2515,12 @@ int pic_create(const pic_mesh_desc *mesh, const pic_params *par, pic_handle **ou
   rc |= dalloc(h, &h->arrCnt, hm.nElems);
   rc |= dalloc(h, &h->insideById, cap);
   rc |= dalloc(h, &h->stateById, cap * 6);
-  rc |= dalloc(h, &h->mv.count, 2);
-  rc |= dalloc(h, &h->mv.idx, cap);
+  rc |= dalloc(h, &h->mv.count, kMoverCounters);
+  h->mv.seg = mover_seg(cap);
+  rc |= dalloc(h, &h->mv.idx, size_t(h->mv.seg) * kMoverSegs);
   rc |= dalloc(h, &h->mv.last, cap * 3);
   if (par->tracking == PIC_TRACK_REFMAPPING) {
-    rc |= dalloc(h, &h->mv.flag, cap);
-    rc |= dalloc(h, &h->mv.slot2, cap);
+    rc |= dalloc(h, &h->mv.late, cap);
   }
   rc |= dalloc(h, &h->lostCount, 1);
   if (rc) { pic_destroy(h); return PIC_EHIP; }
@@ -2527,7 +2531,7 @@ int pic_create(const pic_mesh_desc *mesh, const pic_params *par, pic_handle **ou
   *h->hostTotal = 0;
   // counters that the end of every sort clears again
   HIPCHK(hipMemset(h->arrCnt, 0, size_t(hm.nElems) * sizeof(int32_t)));
-  HIPCHK(hipMemset(h->mv.count, 0, 2 * sizeof(int32_t)));
+  HIPCHK(hipMemset(h->mv.count, 0, kMoverCounters * sizeof(int32_t)));
   HIPCHK(hipMemset(h->lostCount, 0, sizeof(unsigned long long)));
   HIPCHK(hipMemset(h->E, 0, size_t(hm.nElems) * hm.nDof * 3 * sizeof(double)));
   HIPCHK(hipMemset(h->PS, 0, size_t(hm.nElems) * hm.nDof * 4 * sizeof(double)));
@@ -2744,8 +2748,8 @@ int pic_perform_tracking(pic_handle *h) {
     } else {
       auto kt = h->M.affine ? k_track_inside<true> : k_track_inside<false>;
       hipLaunchKernelGGL(kt, dim3(grid_for(h->n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->n, h->newElem, h->mv);
-      hipLaunchKernelGGL(k_track_movers<true>, dim3(1024), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
-                         h->lostCount, h->insideById, h->stateById);
+      hipLaunchKernelGGL(k_track_movers<true>, dim3(mover_grid(h->n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem,
+                         h->mv, h->lostCount, h->insideById, h->stateById);
     }
     HIPCHK(hipGetLastError());
     if (int rc = run_sort(h, true)) return rc;
@@ -2769,6 +2773,7 @@ int enqueue_step(pic_handle *h, double dt, int64_t nGrid, bool timed) {
   const int32_t *nDev = h->start + ne;
   const bool mixed = h->par.precision == PIC_PREC_MIXED;   // N = 3
   const dim3 grid(grid_for(std::max<int64_t>(nGrid, 1)));
+  const dim3 moverGrid(mover_grid(nGrid));
   if (h->par.tracking == PIC_TRACK_REFMAPPING) {
     if (mixed && h->hm.NGeo == 1)
       hipLaunchKernelGGL((k_rm_push_inside<3, 2, true>), grid, dim3(kBlock), 0, h->stream, h->M, h->P, nGrid, dt,
@@ -2779,8 +2784,8 @@ int enqueue_step(pic_handle *h, double dt, int64_t nGrid, bool timed) {
     else
       LAUNCH_NG(k_rm_push_inside, h->hm.N, h->hm.NGeo, grid, h->M, h->P, nGrid, dt, h->newElem, h->mv, nDev);
     if (timed) HIPCHK(hipEventRecord(h->ev[kEvPush], h->stream));
-    LAUNCH_NG(k_rm_movers, h->hm.N, h->hm.NGeo, dim3(std::min<unsigned>(grid.x, 4096u)), h->M, h->P, h->newElem, h->mv,
-              h->lostCount, h->insideById, h->stateById);
+    LAUNCH_NG(k_rm_movers, h->hm.N, h->hm.NGeo, moverGrid, h->M, h->P, h->newElem, h->mv, h->lostCount,
+              h->insideById, h->stateById);
     if (h->hm.nBC > 0)
       LAUNCH_NG(k_rm_bc_movers, h->hm.N, h->hm.NGeo, dim3(1024), h->M, h->P, h->newElem, h->mv, h->lostCount,
                 h->insideById, h->stateById);
@@ -2795,7 +2800,7 @@ int enqueue_step(pic_handle *h, double dt, int64_t nGrid, bool timed) {
     else if (aff) { LAUNCH_N3(k_push_inside, h->hm.N, false, true, grid, h->M, h->P, nGrid, dt, h->newElem, h->mv, nDev); }
     else { LAUNCH_N(k_push_inside, h->hm.N, grid, h->M, h->P, nGrid, dt, h->newElem, h->mv, nDev); }
     if (timed) HIPCHK(hipEventRecord(h->ev[kEvPush], h->stream));
-    hipLaunchKernelGGL(k_track_movers<false>, dim3(1024), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
+    hipLaunchKernelGGL(k_track_movers<false>, moverGrid, dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem, h->mv,
                        h->lostCount, h->insideById, h->stateById);
   }
   HIPCHK(hipGetLastError());
