@@ -247,9 +247,9 @@ int emit_impl(pic_handle *h, int32_t n_inits, const pic_emission *inits, uint64_
     hipLaunchKernelGGL(k_emit, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, A, n, state, xyz, elem, spec);
     // SinglePointToElement on the device
     if (h->par.tracking == PIC_TRACK_REFMAPPING) {
-      LAUNCH_NG(k_rm_locate, h->hm.N, h->hm.NGeo, dim3(grid_for(n)), h->M, n, xyz, elem);
+      LAUNCH_NG(k_rm_locate, h->hm.N, h->hm.NGeo, dim3(grid_for(n)), h->M, n, xyz, 3, elem);
     } else {
-      hipLaunchKernelGGL(k_tria_locate, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, h->M, n, xyz, elem);
+      hipLaunchKernelGGL(k_tria_locate, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, h->M, n, xyz, 3, elem);
     }
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(h->stream) != hipSuccess ||
         hipMemcpy(hs.data(), state, size_t(n) * 6 * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess ||

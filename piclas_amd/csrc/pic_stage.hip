@@ -125,7 +125,7 @@ struct Movers {
   int32_t *idx;     // [kMoverSegs][seg] particles
   int64_t seg;      // places per segment
   int32_t *late;    // [cap] RefMapping: the particles that k_rm_movers passes on
-  double *last;     // [cap][3] positions of particles to be located (set-up)
+  double *last;     // [cap][3] positions of particles to be checked (restart)
 };
 // places per segment: all particles of the workgroups that share it
 inline int64_t mover_seg(int64_t cap) { return ((cap + kBlock - 1) / kBlock + kMoverSegs - 1) / kMoverSegs * kBlock; }
@@ -484,21 +484,24 @@ __global__ __launch_bounds__(kBlock) void k_rm_init(DevMesh M, DevParts P, int64
   P.rx[i] = xi[0]; P.ry[i] = xi[1]; P.rz[i] = xi[2];
 }
 
-// SinglePointToElement for particles handed over without an element
+// SinglePointToElement for particles handed over without an element (elem -1;
+// xyz: their positions, stride doubles apart)
 template <int N, int G>
-__global__ __launch_bounds__(kBlock) void k_rm_locate(DevMesh M, int64_t n, const double *xyz, int32_t *elem) {
+__global__ __launch_bounds__(kBlock) void k_rm_locate(DevMesh M, int64_t n, const double *xyz, int stride,
+                                                       int32_t *elem) {
   const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   if (i >= n) return;
-  if (elem[i] >= 0) return;
-  const double x[3] = {xyz[i * 3], xyz[i * 3 + 1], xyz[i * 3 + 2]};
+  if (elem[i] != -1) return;
+  const double x[3] = {xyz[i * stride], xyz[i * stride + 1], xyz[i * stride + 2]};
   double xi[3];
   elem[i] = rm_locate<N, G>(M, x, xi);
 }
-__global__ __launch_bounds__(kBlock) void k_tria_locate(DevMesh M, int64_t n, const double *xyz, int32_t *elem) {
+__global__ __launch_bounds__(kBlock) void k_tria_locate(DevMesh M, int64_t n, const double *xyz, int stride,
+                                                       int32_t *elem) {
   const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   if (i >= n) return;
-  if (elem[i] >= 0) return;
-  const double x[3] = {xyz[i * 3], xyz[i * 3 + 1], xyz[i * 3 + 2]};
+  if (elem[i] != -1) return;
+  const double x[3] = {xyz[i * stride], xyz[i * stride + 1], xyz[i * stride + 2]};
   elem[i] = tria_locate(M, x);
 }
 
@@ -558,7 +561,7 @@ __global__ __launch_bounds__(kBlock) void k_seg_rank(int nElems, const int32_t *
   if (lane == 0) stayCnt[w] = stay;
 }
 
-// exclusive scan of stayCnt+arrCnt into newStart[0..nElems], single
+// exclusive scan of stayCnt+arrCnt (arrCnt may be null) into newStart[0..nElems], single
 // workgroup: tiles of 4096 counts, 4 consecutive per thread (one 16-byte
 // load each), wave scans, wave totals through LDS, the next tile's loads in
 // flight during the current tile's scan.
@@ -567,14 +570,16 @@ __global__ __launch_bounds__(1024) void k_scan(int nElems, const int32_t *stayCn
   const int t = threadIdx.x, lane = lane_id(), w = t / kWave;
   auto load4 = [&](int base, int4 &a, int4 &b) {
     const int e = base + 4 * t;
+    b = make_int4(0, 0, 0, 0);
     if (e + 3 < nElems) {
       a = *reinterpret_cast<const int4 *>(stayCnt + e);
-      b = *reinterpret_cast<const int4 *>(arrCnt + e);
+      if (arrCnt) b = *reinterpret_cast<const int4 *>(arrCnt + e);
     } else {
       a = make_int4(e < nElems ? stayCnt[e] : 0, e + 1 < nElems ? stayCnt[e + 1] : 0,
                     e + 2 < nElems ? stayCnt[e + 2] : 0, 0);
-      b = make_int4(e < nElems ? arrCnt[e] : 0, e + 1 < nElems ? arrCnt[e + 1] : 0,
-                    e + 2 < nElems ? arrCnt[e + 2] : 0, 0);
+      if (arrCnt)
+        b = make_int4(e < nElems ? arrCnt[e] : 0, e + 1 < nElems ? arrCnt[e + 1] : 0,
+                      e + 2 < nElems ? arrCnt[e + 2] : 0, 0);
     }
   };
   int carry = 0;
@@ -722,6 +727,130 @@ __global__ __launch_bounds__(kBlock) void k_gather_state(const int32_t *total, c
     }
   }
   if (blk) record_block_box(blk, j, valid && f != 0.0, x, y, z);
+}
+
+// ---- hand-over of particles -------------------------------------------------
+// pic_set_particles and pic_get_particles move the caller's arrays as they
+// are and order them on the device (on the host, one thread, the loops over a
+// million particles took 46 of a hand-over's 53 ms).
+
+// 0-based elements (-1: to be located, -2: marked as outside) and species;
+// bad: 2 i for the first element, 2 i + 1 for the first species out of range
+__global__ __launch_bounds__(kBlock) void k_set_check(int64_t n, int nElems, int nSpecies, bool outsideMarked,
+                                                      const int32_t *elemIn, const int32_t *specIn, int32_t *elem,
+                                                      uint8_t *spec, unsigned long long *bad) {
+  const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const int e = elemIn ? elemIn[i] : 0, sp = specIn ? specIn[i] - 1 : 0;
+  const bool outside = outsideMarked && e == -1;
+  if (!outside && (e < 0 || e > nElems)) atomicMin(bad, (unsigned long long)(2 * i));
+  if (sp < 0 || sp >= nSpecies) atomicMin(bad, (unsigned long long)(2 * i + 1));
+  elem[i] = outside ? -2 : e - 1;
+  spec[i] = uint8_t(sp);
+}
+
+// One pass of a stable radix sort by 8 bits of the element (particles without
+// one count as element nElems and go last): per tile of 4096 keys the counts
+// of the 256 digits, their scan in digit-major order, and the move, each wave
+// taking its quarter of the tile in order and ranking 64 keys at a time by
+// ballots.  idxIn null: the first pass, key i is particle i.
+constexpr int kRadixTile = 4096, kRadixBins = 256;
+__device__ inline int sort_key(int e, int nElems) { return e < 0 ? nElems : e; }
+__global__ __launch_bounds__(kBlock) void k_radix_count(int64_t n, int nElems, const int32_t *key, int bit, int32_t *cnt) {
+  __shared__ int32_t c[kRadixBins];
+  c[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t base = int64_t(blockIdx.x) * kRadixTile;
+  for (int q = threadIdx.x; q < kRadixTile && base + q < n; q += kBlock)
+    atomicAdd(&c[(sort_key(key[base + q], nElems) >> bit) & (kRadixBins - 1)], 1);
+  __syncthreads();
+  cnt[int64_t(threadIdx.x) * gridDim.x + blockIdx.x] = c[threadIdx.x];
+}
+__global__ __launch_bounds__(kBlock) void k_radix_move(int64_t n, int nElems, const int32_t *key, const int32_t *idxIn,
+                                                       int bit, const int32_t *off, int32_t *keyOut, int32_t *idxOut) {
+  constexpr int nw = kBlock / kWave, part = kRadixTile / nw;
+  __shared__ int32_t at[nw][kRadixBins];
+  const int wib = threadIdx.x / kWave, lane = lane_id();
+  for (int w = 0; w < nw; ++w) at[w][threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t base = int64_t(blockIdx.x) * kRadixTile + wib * part;
+  for (int q = lane; q < part && base + q < n; q += kWave)
+    atomicAdd(&at[wib][(sort_key(key[base + q], nElems) >> bit) & (kRadixBins - 1)], 1);
+  __syncthreads();
+  int run = off[int64_t(threadIdx.x) * gridDim.x + blockIdx.x];
+  for (int w = 0; w < nw; ++w) {
+    const int c = at[w][threadIdx.x];
+    at[w][threadIdx.x] = run;
+    run += c;
+  }
+  __syncthreads();
+  for (int q = 0; q < part && base + q < n; q += kWave) {
+    const int64_t i = base + q + lane;
+    const bool valid = i < n;
+    const int k = valid ? sort_key(key[i], nElems) : 0, d = (k >> bit) & (kRadixBins - 1);
+    unsigned long long m = __ballot(valid);   // the lanes with this lane's digit
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const unsigned long long one = __ballot(valid && ((d >> b) & 1));
+      m &= (d >> b) & 1 ? one : ~one;
+    }
+    const unsigned long long below = m & ((1ull << lane) - 1ull);
+    const int pos = at[wib][d] + __popcll(below);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (valid) {
+      if (below == 0) at[wib][d] = pos + __popcll(m);   // the first of its lanes
+      keyOut[pos] = k;
+      idxOut[pos] = idxIn ? idxIn[i] : int32_t(i);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// segment offsets from the sorted keys, and the particle count to the host
+__global__ __launch_bounds__(kBlock) void k_set_start(int64_t n, int nElems, const int32_t *key, int32_t *start,
+                                                      int32_t *hostTotal) {
+  const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (j > n) return;
+  const int k = j < n ? key[j] : nElems, prev = j > 0 ? key[j - 1] : -1;
+  for (int e = prev + 1; e <= k; ++e) start[e] = int32_t(j);
+  if (prev < nElems && k == nElems) *hostTotal = int32_t(j);
+}
+
+// the sorted arrays; the state of a particle that no element holds is kept by id
+__global__ __launch_bounds__(kBlock) void k_set_state(int64_t n, int nElems, const int32_t *key, const int32_t *idx,
+                                                      const double *state, const uint8_t *spec, const uint8_t *isNew,
+                                                      DevParts P, uint8_t *insideById, double *stateById) {
+  const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (j >= n) return;
+  const int i = idx[j], e = key[j];
+  const double *st = state + int64_t(i) * 6;
+  insideById[i] = e < nElems;
+  if (e < nElems) {
+    P.x[j] = st[0]; P.y[j] = st[1]; P.z[j] = st[2];
+    P.vx[j] = st[3]; P.vy[j] = st[4]; P.vz[j] = st[5];
+    P.elem[j] = e; P.id[j] = i; P.spec[j] = spec[i]; P.isNew[j] = isNew ? isNew[i] : 0;
+  } else {
+    for (int c = 0; c < 6; ++c) stateById[int64_t(i) * 6 + c] = st[c];
+  }
+}
+
+// PartState rows and 1-based elements (0: not inside) in the caller's order
+__global__ __launch_bounds__(kBlock) void k_get_particles(int64_t n, int64_t nTotal, DevParts P, const uint8_t *insideById,
+                                                          const double *stateById, double *state, int32_t *elem) {
+  const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (j < n) {
+    const int64_t i = P.id[j];
+    double *st = state + i * 6;
+    st[0] = P.x[j]; st[1] = P.y[j]; st[2] = P.z[j];
+    st[3] = P.vx[j]; st[4] = P.vy[j]; st[5] = P.vz[j];
+    elem[i] = P.elem[j] + 1;
+  }
+  if (j < nTotal && !insideById[j]) {
+    for (int c = 0; c < 6; ++c) state[j * 6 + c] = stateById[j * 6 + c];
+    elem[j] = 0;
+  }
 }
 
 // ---- cell_volweight_mean ----------------------------------------------------
@@ -1931,7 +2060,9 @@ struct pic_handle {
   const double *graphP = nullptr;
   Movers mv{};
   bool stagedValid = false;   // LastPartPos/FieldAtParticle refer to the current order
-  std::vector<std::pair<int64_t, std::vector<double>>> unplaced;  // particles no element holds at set-up
+  // hand-over: first bad entry, digit counts and offsets of the radix sort
+  unsigned long long *setBad = nullptr;
+  int32_t *radixCnt = nullptr, *radixOff = nullptr;
   // statistics
   // device times of an eager step: one event per boundary that the statistics
   // read (every record costs host time and a packet between two kernels)
@@ -2523,6 +2654,10 @@ int pic_create(const pic_mesh_desc *mesh, const pic_params *par, pic_handle **ou
     rc |= dalloc(h, &h->mv.late, cap);
   }
   rc |= dalloc(h, &h->lostCount, 1);
+  rc |= dalloc(h, &h->setBad, 1);
+  const size_t radix = size_t((cap + kRadixTile - 1) / kRadixTile) * kRadixBins;
+  rc |= dalloc(h, &h->radixCnt, radix);
+  rc |= dalloc(h, &h->radixOff, radix + 1);
   if (rc) { pic_destroy(h); return PIC_EHIP; }
   if (hipHostMalloc(&h->hostTotal, 64, hipHostMallocDefault) != hipSuccess) {
     pic_destroy(h);
@@ -2601,79 +2736,49 @@ int set_particles_impl(pic_handle *h, int64_t n, const double *PartState, const 
   if (n < 0 || n > h->cap) return fail(PIC_ECAPACITY, "pic_set_particles: more particles than max_particles");
   if (set_device(h)) return PIC_EHIP;
   const int ne = h->hm.nElems;
-  std::vector<int32_t> el(n), sp(n, 0);
-  std::vector<uint8_t> ins(n, 1);
   const bool refmap = h->par.tracking == PIC_TRACK_REFMAPPING;
-  std::vector<int64_t> pending;
-  for (int64_t i = 0; i < n; ++i) {
-    int e = elem ? elem[i] : 0;
-    if (outsideMarked && e == -1) {
-      el[i] = -1;
-    } else {
-      if (e < 0 || e > ne) return fail(PIC_EINVAL, "pic_set_particles: element id out of range");
-      if (e == 0) pending.push_back(i);
-      el[i] = e - 1;
-    }
-    sp[i] = species ? species[i] - 1 : 0;
-    if (sp[i] < 0 || sp[i] >= h->par.nSpecies) return fail(PIC_EINVAL, "pic_set_particles: species out of range");
+  // Into scratch arrays first: a call that fails leaves the particles as they are.
+  double *state = h->Q.F;
+  auto put = [&](void *dst, const void *src, size_t bytes) {
+    return bytes == 0 || !src ? hipSuccess : hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream);
+  };
+  HIPCHK(put(state, PartState, size_t(n) * 6 * sizeof(double)));
+  HIPCHK(put(h->newElem, elem, size_t(n) * sizeof(int32_t)));
+  HIPCHK(put(h->rank, species, size_t(n) * sizeof(int32_t)));
+  HIPCHK(put(h->Q.isNew, is_new, size_t(n)));
+  const dim3 grid(grid_for(std::max<int64_t>(n, 1)));
+  HIPCHK(hipMemsetAsync(h->setBad, 0xff, sizeof(unsigned long long), h->stream));
+  hipLaunchKernelGGL(k_set_check, grid, dim3(kBlock), 0, h->stream, n, ne, h->par.nSpecies, outsideMarked,
+                     elem ? h->newElem : nullptr, species ? h->rank : nullptr, h->newElem, h->Q.spec, h->setBad);
+  // SinglePointToElement on the device for the particles without an element
+  if (refmap) { LAUNCH_NG(k_rm_locate, h->hm.N, h->hm.NGeo, grid, h->M, n, state, 6, h->newElem); }
+  else hipLaunchKernelGGL(k_tria_locate, grid, dim3(kBlock), 0, h->stream, h->M, n, state, 6, h->newElem);
+  HIPCHK(hipGetLastError());
+  unsigned long long bad = 0;
+  HIPCHK(hipMemcpyAsync(&bad, h->setBad, sizeof(bad), hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(hipStreamSynchronize(h->stream));
+  if (bad != ~0ull)
+    return fail(PIC_EINVAL, bad % 2 == 0 ? "pic_set_particles: element id out of range" : "pic_set_particles: species out of range");
+  // stable sort by element: the caller's order within one
+  const int tiles = int(std::max<int64_t>(1, (n + kRadixTile - 1) / kRadixTile));
+  const int32_t *key = h->newElem, *idx = nullptr;
+  for (int bit = 0; bit == 0 || (ne >> bit) > 0; bit += 8) {
+    int32_t *keyOut = (bit / 8) % 2 == 0 ? h->rank : h->Q.elem, *idxOut = (bit / 8) % 2 == 0 ? h->arr : h->Q.id;
+    hipLaunchKernelGGL(k_radix_count, dim3(tiles), dim3(kBlock), 0, h->stream, n, ne, key, bit, h->radixCnt);
+    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, h->stream, kRadixBins * tiles, h->radixCnt,
+                       static_cast<const int32_t *>(nullptr), h->radixOff);
+    hipLaunchKernelGGL(k_radix_move, dim3(tiles), dim3(kBlock), 0, h->stream, n, ne, key, idx, bit, h->radixOff, keyOut,
+                       idxOut);
+    key = keyOut;
+    idx = idxOut;
   }
-  if (!pending.empty()) {
-    // SinglePointToElement on the device for the particles without an element
-    const int64_t np = int64_t(pending.size());
-    std::vector<double> xyz(np * 3);
-    std::vector<int32_t> pe(np, -1);
-    for (int64_t k = 0; k < np; ++k)
-      for (int c = 0; c < 3; ++c) xyz[k * 3 + c] = PartState[pending[k] * 6 + c];
-    HIPCHK(copy_bytes(h->mv.last, xyz.data(), np * 3 * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(copy_bytes(h->newElem, pe.data(), np * sizeof(int32_t), hipMemcpyHostToDevice));
-    if (refmap) { LAUNCH_NG(k_rm_locate, h->hm.N, h->hm.NGeo, dim3(grid_for(np)), h->M, np, h->mv.last, h->newElem); }
-    else hipLaunchKernelGGL(k_tria_locate, dim3(grid_for(np)), dim3(kBlock), 0, h->stream, h->M, np, h->mv.last, h->newElem);
-    HIPCHK(hipGetLastError());
-    // the stage's stream does not synchronise with the null stream's copies
-    HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(copy_bytes(pe.data(), h->newElem, np * sizeof(int32_t), hipMemcpyDeviceToHost));
-    for (int64_t k = 0; k < np; ++k) el[pending[k]] = pe[k];
-  }
-  for (int64_t i = 0; i < n; ++i)
-    if (el[i] < 0) ins[i] = 0;
-  // counting sort by element, stable in caller order
-  std::vector<int64_t> cnt(ne + 1, 0);
-  for (int64_t i = 0; i < n; ++i)
-    if (el[i] >= 0) cnt[el[i] + 1]++;
-  for (int e = 0; e < ne; ++e) cnt[e + 1] += cnt[e];
-  const int64_t nin = cnt[ne];
-  std::vector<int32_t> start(ne + 1);
-  for (int e = 0; e <= ne; ++e) start[e] = int32_t(cnt[e]);
-  std::vector<int64_t> order(nin);
-  {
-    std::vector<int64_t> fill(cnt.begin(), cnt.end() - 1);
-    for (int64_t i = 0; i < n; ++i)
-      if (el[i] >= 0) order[fill[el[i]]++] = i;
-  }
-  std::vector<double> buf(nin);
-  double *dst[6] = {h->P.x, h->P.y, h->P.z, h->P.vx, h->P.vy, h->P.vz};
-  for (int c = 0; c < 6; ++c) {
-    for (int64_t j = 0; j < nin; ++j) buf[j] = PartState[order[j] * 6 + c];
-    HIPCHK(copy_bytes(dst[c], buf.data(), nin * sizeof(double), hipMemcpyHostToDevice));
-  }
-  std::vector<int32_t> ib(nin);
-  std::vector<uint8_t> ub(nin);
-  for (int64_t j = 0; j < nin; ++j) ib[j] = el[order[j]];
-  HIPCHK(copy_bytes(h->P.elem, ib.data(), nin * sizeof(int32_t), hipMemcpyHostToDevice));
-  for (int64_t j = 0; j < nin; ++j) ib[j] = int32_t(order[j]);
-  HIPCHK(copy_bytes(h->P.id, ib.data(), nin * sizeof(int32_t), hipMemcpyHostToDevice));
-  for (int64_t j = 0; j < nin; ++j) ub[j] = uint8_t(sp[order[j]]);
-  HIPCHK(copy_bytes(h->P.spec, ub.data(), nin, hipMemcpyHostToDevice));
-  for (int64_t j = 0; j < nin; ++j) ub[j] = is_new ? is_new[order[j]] : 0;
-  HIPCHK(copy_bytes(h->P.isNew, ub.data(), nin, hipMemcpyHostToDevice));
-  HIPCHK(copy_bytes(h->start, start.data(), (ne + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
-  HIPCHK(copy_bytes(h->insideById, ins.data(), n, hipMemcpyHostToDevice));
-  HIPCHK(hipMemset(h->lostCount, 0, sizeof(unsigned long long)));
-  // particles no element holds keep their state for pic_get_particles
-  h->unplaced.clear();
-  for (int64_t i = 0; i < n; ++i)
-    if (!ins[i]) h->unplaced.emplace_back(i, std::vector<double>(PartState + i * 6, PartState + i * 6 + 6));
-  h->n = nin;
+  hipLaunchKernelGGL(k_set_start, dim3(grid_for(n + 1)), dim3(kBlock), 0, h->stream, n, ne, key, h->start, h->hostTotal);
+  hipLaunchKernelGGL(k_set_state, grid, dim3(kBlock), 0, h->stream, n, ne, key, idx, state, h->Q.spec,
+                     is_new ? h->Q.isNew : nullptr, h->P, h->insideById, h->stateById);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemsetAsync(h->lostCount, 0, sizeof(unsigned long long), h->stream));
+  if (int rc = read_count(h)) return rc;
+  const int64_t nin = h->n;
   h->nTotal = n;
   h->particlesSet = true;
   h->stagedValid = false;
@@ -2681,7 +2786,7 @@ int set_particles_impl(pic_handle *h, int64_t n, const double *PartState, const 
   if (refmap && nin > 0) {
     LAUNCH_NG(k_rm_init, h->hm.N, h->hm.NGeo, dim3(grid_for(nin)), h->M, h->P, nin);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipDeviceSynchronize());
+    HIPCHK(hipStreamSynchronize(h->stream));
   }
   return PIC_OK;
 }
@@ -2913,36 +3018,17 @@ int pic_get_particles(pic_handle *h, double *PartState, int32_t *elem, uint8_t *
   if (set_device(h)) return PIC_EHIP;
   HIPCHK(hipStreamSynchronize(h->stream));
   const int64_t n = h->n, nt = h->nTotal;
-  std::vector<double> a(n);
-  std::vector<int32_t> id(n), el(n);
-  std::vector<uint8_t> ins(nt);
-  HIPCHK(copy_bytes(id.data(), h->P.id, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-  HIPCHK(copy_bytes(el.data(), h->P.elem, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-  HIPCHK(copy_bytes(ins.data(), h->insideById, nt, hipMemcpyDeviceToHost));
-  if (PartState) {
-    double *src[6] = {h->P.x, h->P.y, h->P.z, h->P.vx, h->P.vy, h->P.vz};
-    for (int c = 0; c < 6; ++c) {
-      HIPCHK(copy_bytes(a.data(), src[c], n * sizeof(double), hipMemcpyDeviceToHost));
-      for (int64_t j = 0; j < n; ++j) PartState[int64_t(id[j]) * 6 + c] = a[j];
-    }
-    int64_t nlost = 0;
-    for (int64_t i = 0; i < nt; ++i) nlost += ins[i] ? 0 : 1;
-    if (nlost > 0) {
-      std::vector<double> st(size_t(nt) * 6);
-      HIPCHK(copy_bytes(st.data(), h->stateById, size_t(nt) * 6 * sizeof(double), hipMemcpyDeviceToHost));
-      for (int64_t i = 0; i < nt; ++i)
-        if (!ins[i])
-          for (int c = 0; c < 6; ++c) PartState[i * 6 + c] = st[i * 6 + c];
-      for (auto &u : h->unplaced)
-        for (int c = 0; c < 6; ++c) PartState[u.first * 6 + c] = u.second[c];
-    }
-  }
-  if (elem) {
-    for (int64_t i = 0; i < nt; ++i) elem[i] = 0;
-    for (int64_t j = 0; j < n; ++j) elem[id[j]] = el[j] + 1;
-  }
-  if (inside)
-    for (int64_t i = 0; i < nt; ++i) inside[i] = ins[i];
+  if (nt == 0) return PIC_OK;
+  hipLaunchKernelGGL(k_get_particles, dim3(grid_for(nt)), dim3(kBlock), 0, h->stream, n, nt, h->P, h->insideById,
+                     h->stateById, h->Q.F, h->newElem);
+  HIPCHK(hipGetLastError());
+  auto get = [&](void *dst, const void *src, size_t bytes) {
+    return dst ? hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream) : hipSuccess;
+  };
+  HIPCHK(get(PartState, h->Q.F, size_t(nt) * 6 * sizeof(double)));
+  HIPCHK(get(elem, h->newElem, size_t(nt) * sizeof(int32_t)));
+  HIPCHK(get(inside, h->insideById, size_t(nt)));
+  HIPCHK(hipStreamSynchronize(h->stream));
   return PIC_OK;
 }
 

@@ -97,8 +97,8 @@ int pic_restart_particles(pic_handle *h, int64_t n, const double *PartData, cons
     HIPCHK(copy_bytes(chk.data(), h->newElem, size_t(n) * sizeof(int32_t), hipMemcpyDeviceToHost));
     for (int64_t p = 0; p < n; ++p) missing += chk[p] < 0;
     if (missing > 0) {
-      if (refmap) { LAUNCH_NG(k_rm_locate, h->hm.N, h->hm.NGeo, dim3(grid_for(n)), h->M, n, h->mv.last, h->newElem); }
-      else hipLaunchKernelGGL(k_tria_locate, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, h->M, n, h->mv.last,
+      if (refmap) { LAUNCH_NG(k_rm_locate, h->hm.N, h->hm.NGeo, dim3(grid_for(n)), h->M, n, h->mv.last, 3, h->newElem); }
+      else hipLaunchKernelGGL(k_tria_locate, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, h->M, n, h->mv.last, 3,
                               h->newElem);
       HIPCHK(hipGetLastError());
       HIPCHK(hipStreamSynchronize(h->stream));
