@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_sf_cart(DevMesh M, DevParts P, i
         double si1 = 0.0, six = 0.0;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const double S = fmax(D - s2[c], 0.0);
+          const double S = clamp01(D - s2[c]);   // (S <= 1: the clamp is free)
           double Sa = S;   // S^(alpha-1)
           if (ALPHA == 0) {
             for (int ex = 3; ex <= A.alpha; ++ex) Sa = Sa * S;

@@ -621,7 +621,8 @@ __global__ __launch_bounds__(1024) void k_scan(int nElems, const int32_t *stayCn
 
 // The sorted slot of every particle: perm[slot] = old index for the particles
 // that stay, arr[slot] for the arrivals (the sign of rank tells them apart),
-// whose slots k_fix_arrivals puts in order.
+// whose slots are put in order by k_fix_arrivals, or (arr = perm) by
+// k_gather_state.
 __global__ __launch_bounds__(kBlock) void k_dest(int64_t n, const int32_t *newElem, const int32_t *rank,
                                                  const int32_t *newStart, const int32_t *stayCnt, int32_t *perm,
                                                  int32_t *arr, const int32_t *nDev) {
@@ -639,6 +640,7 @@ __global__ __launch_bounds__(kBlock) void k_dest(int64_t n, const int32_t *newEl
 // element, each counting for its arrivals the smaller ids (an insertion sort
 // by one thread took 36 us where some tens arrive per element, now 11).
 constexpr int kFixLanes = 8;
+constexpr int64_t kFixInGather = int64_t(1) << 20;   // particles up to which k_gather_state does it
 __global__ __launch_bounds__(kBlock) void k_fix_arrivals(int nElems, const int32_t *newStart, const int32_t *stayCnt,
                                                          const int32_t *arrCnt, const int32_t *id, const int32_t *arr,
                                                          int32_t *perm) {
@@ -691,12 +693,18 @@ struct SortEnd {
   int nElems;
   int32_t *arrCnt, *moverCount, *hostTotal;
 };
-// STAGED: LastPartPos, LastElem and FieldAtParticle move too
-template <bool STAGED>
+// STAGED: LastPartPos, LastElem and FieldAtParticle move too.  FIX: the
+// arrivals of an element lie in perm in any order, and the thread of one finds
+// its place among them (its rank by caller id; arrivals are few), which spares
+// the launch of k_fix_arrivals; not where the block boxes are written, as they
+// are reduced over a wave's 64 consecutive slots.
+template <bool STAGED, bool FIX>
 __global__ __launch_bounds__(kBlock) void k_gather_state(const int32_t *total, const int32_t *perm, DevParts s, DevParts d,
-                                                         const int32_t *newElem, SpeciesFactor sf, double4 *rec,
-                                                         double4 *recB, double4 *blk, SortEnd end) {
-  const int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+                                                         const int32_t *newElem, const int32_t *rank,
+                                                         const int32_t *newStart, const int32_t *stayCnt,
+                                                         SpeciesFactor sf, double4 *rec, double4 *recB, double4 *blk,
+                                                         SortEnd end) {
+  int64_t j = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   const int64_t n = *total;
   for (int64_t e = j; e < end.nElems; e += int64_t(gridDim.x) * kBlock) end.arrCnt[e] = 0;
   for (int64_t e = j; e < kMoverCounters; e += int64_t(gridDim.x) * kBlock) end.moverCount[e] = 0;
@@ -706,13 +714,20 @@ __global__ __launch_bounds__(kBlock) void k_gather_state(const int32_t *total, c
   double x = 0.0, y = 0.0, z = 0.0, f = 0.0;
   if (valid) {
     const int32_t i = perm[j];
+    const int32_t ne = newElem[i];
+    if (FIX && rank[i] < 0) {
+      const int b = newStart[ne] + stayCnt[ne], na = newStart[ne + 1] - b, key = s.id[i];
+      int r = 0;
+      for (int k = 0; k < na; ++k) r += s.id[perm[b + k]] < key;
+      j = b + r;
+    }
     x = s.x[i]; y = s.y[i]; z = s.z[i];
     const double vx = s.vx[i], vy = s.vy[i], vz = s.vz[i];
     const uint8_t sp = s.spec[i];
     d.x[j] = x; d.y[j] = y; d.z[j] = z;
     d.vx[j] = vx; d.vy[j] = vy; d.vz[j] = vz;
     d.id[j] = s.id[i]; d.spec[j] = sp; d.isNew[j] = s.isNew[i];
-    d.elem[j] = newElem[i];
+    d.elem[j] = ne;
     if (s.rx) { d.rx[j] = s.rx[i]; d.ry[j] = s.ry[i]; d.rz[j] = s.rz[i]; }
     if (STAGED) {
       d.lx[j] = s.lx[i]; d.ly[j] = s.ly[i]; d.lz[j] = s.lz[i];
@@ -2335,20 +2350,26 @@ int enqueue_sort(pic_handle *h, int64_t nGrid, bool withStaged) {
   hipLaunchKernelGGL(k_seg_rank, dim3(grid_for(int64_t(ne) * kWave)), dim3(kBlock), 0, h->stream, ne, h->start,
                      h->newElem, h->P.z, h->M.xGPe, h->hm.nDof, h->stayCnt, h->arrCnt, h->rank);
   hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, h->stream, ne, h->stayCnt, h->arrCnt, h->startNew);
-  hipLaunchKernelGGL(k_dest, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, n, h->newElem, h->rank, h->startNew,
-                     h->stayCnt, h->perm, h->arr, nOld);
-  hipLaunchKernelGGL(k_fix_arrivals, dim3(grid_for(int64_t(ne) * kFixLanes)), dim3(kBlock), 0, h->stream, ne, h->startNew,
-                     h->stayCnt, h->arrCnt, h->P.id, h->arr, h->perm);
-  const int32_t *total = h->startNew + ne;
   // records for the shape-function gathers that read them
   const bool useRec = h->sf.rec && (h->sfMatrix || h->par.precision == PIC_PREC_MIXED);
+  double4 *blk = useRec ? block_boxes(h) : nullptr;
+  // (same order either way; the launch spared is 3 us, the rank read by every
+  // thread 36 us at 22 million particles)
+  const bool fix = blk == nullptr && n <= kFixInGather;
+  hipLaunchKernelGGL(k_dest, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, n, h->newElem, h->rank, h->startNew,
+                     h->stayCnt, h->perm, fix ? h->perm : h->arr, nOld);
+  if (!fix)
+    hipLaunchKernelGGL(k_fix_arrivals, dim3(grid_for(int64_t(ne) * kFixLanes)), dim3(kBlock), 0, h->stream, ne,
+                       h->startNew, h->stayCnt, h->arrCnt, h->P.id, h->arr, h->perm);
+  const int32_t *total = h->startNew + ne;
   SpeciesFactor sfac{};
   for (int k = 0; k < 8; ++k) sfac.fsp[k] = h->sf.fsp[k];
   const SortEnd end = {ne, h->arrCnt, h->mv.count, h->hostTotal};
-  auto kg = withStaged ? k_gather_state<true> : k_gather_state<false>;
-  hipLaunchKernelGGL(kg, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, total, h->perm, h->P, h->Q, h->newElem, sfac,
-                     useRec ? const_cast<double4 *>(h->sf.rec) : nullptr,
-                     useRec ? const_cast<double4 *>(h->sf.recB) : nullptr, useRec ? block_boxes(h) : nullptr, end);
+  auto kg = withStaged ? (fix ? k_gather_state<true, true> : k_gather_state<true, false>)
+                       : (fix ? k_gather_state<false, true> : k_gather_state<false, false>);
+  hipLaunchKernelGGL(kg, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, total, h->perm, h->P, h->Q, h->newElem, h->rank,
+                     h->startNew, h->stayCnt, sfac, useRec ? const_cast<double4 *>(h->sf.rec) : nullptr,
+                     useRec ? const_cast<double4 *>(h->sf.recB) : nullptr, blk, end);
   if (withStaged) {
     std::swap(h->P.lx, h->Q.lx); std::swap(h->P.ly, h->Q.ly); std::swap(h->P.lz, h->Q.lz);
     std::swap(h->P.lastElem, h->Q.lastElem); std::swap(h->P.F, h->Q.F);
