@@ -264,80 +264,6 @@ __device__ inline const double *uniform_ptr(const double *p) {
   return reinterpret_cast<const double *>((uint64_t(hi) << 32) | uint64_t(lo));
 }
 
-// GetRefNewtonStartValue, interpolation/eval_xyz.f90:498-612 (guesses 1, 2, 4)
-// the 3 coordinates of one point by scalar loads (p wave-uniform; exactly 24 bytes read)
-__device__ inline void sload_xyz(const double *p, double out[3]) {
-  p = uniform_ptr(p);
-  typedef uint32_t dw4 __attribute__((ext_vector_type(4)));
-  typedef uint32_t dw2 __attribute__((ext_vector_type(2)));
-  dw4 a;
-  dw2 b;
-  asm volatile("s_load_dwordx4 %0, %2, 0x0\n\ts_load_dwordx2 %1, %2, 0x10\n\ts_waitcnt lgkmcnt(0)"
-               : "=&s"(a), "=&s"(b) : "s"(p));
-  out[0] = __builtin_bit_cast(double, (uint64_t(a[1]) << 32) | uint64_t(a[0]));
-  out[1] = __builtin_bit_cast(double, (uint64_t(a[3]) << 32) | uint64_t(a[2]));
-  out[2] = __builtin_bit_cast(double, (uint64_t(b[1]) << 32) | uint64_t(b[0]));
-}
-
-// UNI: e is wave-uniform; guess 2 then reads the Gauss points by scalar loads
-template <int N, bool UNI = false>
-__device__ inline void ref_newton_start(const DevMesh &M, int e, const double x[3], double xi[3]) {
-  if (M.refGuess == 1) {
-    const double *b0 = M.bary + (size_t)e * 3;
-    const double P[3] = {x[0] - b0[0], x[1] - b0[1], x[2] - b0[2]};
-    double XL[6];
-#pragma unroll
-    for (int d = 0; d < 6; ++d) {
-      const double *b = M.xiBasis + ((size_t)e * 6 + d) * 3;
-      XL[d] = (P[0] * b[0] + P[1] * b[1] + P[2] * b[2]) * M.slen[(size_t)e * 6 + d];
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) xi[d] = 0.5 * (XL[d] - XL[d + 3]);
-    const double mx = fmax(fabs(xi[0]), fmax(fabs(xi[1]), fabs(xi[2])));
-    if (mx > 1.0 + M.refEps)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) xi[d] = fmax(fmin(1.0, xi[d]), -1.0);
-  } else if (M.refGuess == 2) {
-    constexpr int n1 = N + 1;
-    const double *xg = M.xGPe + (size_t)e * n1 * n1 * n1 * 3;
-    double g[3];
-    if (UNI) sload_xyz(xg, g);
-    else { g[0] = xg[0]; g[1] = xg[1]; g[2] = xg[2]; }
-    const double d0[3] = {x[0] - g[0], x[1] - g[1], x[2] - g[2]};
-    double win = sqrt(d0[0] * d0[0] + d0[1] * d0[1] + d0[2] * d0[2]);
-    xi[0] = xi[1] = xi[2] = M.xGP[0];
-#pragma unroll 1
-    for (int i = 0; i < n1; ++i)
-#pragma unroll 1
-      for (int j = 0; j < n1; ++j)
-#pragma unroll 1
-        for (int k = 0; k < n1; ++k) {
-          const int r = (k * n1 + j) * n1 + i;
-          double dX, dY, dZ;
-          if (UNI) {
-            sload_xyz(xg + r * 3, g);
-            dX = fabs(x[0] - g[0]);
-            if (dX > win) continue;
-            dY = fabs(x[1] - g[1]);
-            if (dY > win) continue;
-            dZ = fabs(x[2] - g[2]);
-            if (dZ > win) continue;
-          } else {
-            dX = fabs(x[0] - xg[r * 3]);
-            if (dX > win) continue;
-            dY = fabs(x[1] - xg[r * 3 + 1]);
-            if (dY > win) continue;
-            dZ = fabs(x[2] - xg[r * 3 + 2]);
-            if (dZ > win) continue;
-          }
-          const double dist = sqrt(dX * dX + dY * dY + dZ * dZ);
-          if (dist < win) { win = dist; xi[0] = M.xGP[i]; xi[1] = M.xGP[j]; xi[2] = M.xGP[k]; }
-        }
-  } else {
-    xi[0] = xi[1] = xi[2] = 0.0;
-  }
-}
-
 // EvaluateFieldAtRefPos with NVar=3 (interpolation/eval_xyz.f90:167-295),
 // summed by factors: U = sum_k L_k sum_j L_j sum_i L_i U_ijk (the reference
 // sums sum_ijk U_ijk L_i (L_j L_k); the two agree to round-off).
@@ -435,6 +361,109 @@ __device__ inline void sload_chunk(const double *p, int c, double buf[16]) {
     sdw2 r;
     asm volatile("s_load_dwordx2 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(r) : "s"(q + k));
     buf[k] = dw_to_d(r[0], r[1]);
+  }
+}
+
+// min(a, b) of two keys: no canonicalisation of the operands first
+__device__ inline double min_key(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// Guess 2 in a wave of one element: the Gauss point nearest to x.  The
+// reference visits the points with the third index fastest and keeps the
+// first of equally near ones.  Here they come in memory order, 16 values per
+// scalar load and wait, and the point's place in the reference's order stands
+// in the last bits of its squared distance, so that one minimum compares
+// both (distances that agree to 2^-43 or better count as equal).  A load and
+// wait per point, the square roots and the early exits had made the push of
+// 6 million particles on a curved mesh (degree 3) 1675 us; so it takes 1494.
+template <int N>
+__device__ inline void nearest_gauss_point_s(const DevMesh &M, int e, const double x[3], double xi[3]) {
+  constexpr int n1 = N + 1, NP = n1 * n1 * 3;
+  constexpr int kBits = 32 - __builtin_clz(n1 * n1 * n1 - 1);
+  constexpr uint32_t kMask = (1u << kBits) - 1;
+  const double *xg = M.xGPe + (size_t)e * n1 * n1 * n1 * 3;
+  double best = HUGE_VAL, d2 = 0.0;
+#pragma unroll 1
+  for (int k = 0; k < n1; ++k) {
+    double near = HUGE_VAL;
+#pragma unroll
+    for (int ch = 0; ch < (NP + 15) / 16; ++ch) {
+      double buf[16];
+      sload_chunk<NP>(xg + k * NP, ch, buf);
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const int v = 16 * ch + q;
+        if (v < NP) {
+          const int c = v % 3, i = (v / 3) % n1, j = v / (3 * n1);
+          const double d = x[c] - buf[q];
+          d2 = c == 0 ? d * d : __builtin_fma(d, d, d2);
+          if (c == 2) {
+            const uint64_t u = __builtin_bit_cast(uint64_t, d2);
+            const uint32_t lo = (uint32_t(u) & ~kMask) | uint32_t((i * n1 + j) * n1);
+            near = min_key(near, dw_to_d(lo, uint32_t(u >> 32)));
+          }
+        }
+      }
+    }
+    const uint64_t u = __builtin_bit_cast(uint64_t, near);
+    best = min_key(best, dw_to_d(uint32_t(u) + uint32_t(k), uint32_t(u >> 32)));
+  }
+  const int at = int(uint32_t(__builtin_bit_cast(uint64_t, best)) & kMask);
+  xi[0] = M.xGP[at / (n1 * n1)];
+  xi[1] = M.xGP[(at / n1) % n1];
+  xi[2] = M.xGP[at % n1];
+}
+
+// GetRefNewtonStartValue, interpolation/eval_xyz.f90:498-612 (guesses 1, 2, 4)
+// UNI: e is wave-uniform; guess 2 then reads the Gauss points by scalar loads
+template <int N, bool UNI = false>
+__device__ inline void ref_newton_start(const DevMesh &M, int e, const double x[3], double xi[3]) {
+  if (M.refGuess == 1) {
+    const double *b0 = M.bary + (size_t)e * 3;
+    const double P[3] = {x[0] - b0[0], x[1] - b0[1], x[2] - b0[2]};
+    double XL[6];
+#pragma unroll
+    for (int d = 0; d < 6; ++d) {
+      const double *b = M.xiBasis + ((size_t)e * 6 + d) * 3;
+      XL[d] = (P[0] * b[0] + P[1] * b[1] + P[2] * b[2]) * M.slen[(size_t)e * 6 + d];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) xi[d] = 0.5 * (XL[d] - XL[d + 3]);
+    const double mx = fmax(fabs(xi[0]), fmax(fabs(xi[1]), fabs(xi[2])));
+    if (mx > 1.0 + M.refEps)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) xi[d] = fmax(fmin(1.0, xi[d]), -1.0);
+  } else if (M.refGuess == 2) {
+    if (UNI) {
+      nearest_gauss_point_s<N>(M, e, x, xi);
+      return;
+    }
+    constexpr int n1 = N + 1;
+    const double *xg = M.xGPe + (size_t)e * n1 * n1 * n1 * 3;
+    const double d0[3] = {x[0] - xg[0], x[1] - xg[1], x[2] - xg[2]};
+    double win = sqrt(d0[0] * d0[0] + d0[1] * d0[1] + d0[2] * d0[2]);
+    xi[0] = xi[1] = xi[2] = M.xGP[0];
+#pragma unroll 1
+    for (int i = 0; i < n1; ++i)
+#pragma unroll 1
+      for (int j = 0; j < n1; ++j)
+#pragma unroll 1
+        for (int k = 0; k < n1; ++k) {
+          const int r = (k * n1 + j) * n1 + i;
+          const double dX = fabs(x[0] - xg[r * 3]);
+          if (dX > win) continue;
+          const double dY = fabs(x[1] - xg[r * 3 + 1]);
+          if (dY > win) continue;
+          const double dZ = fabs(x[2] - xg[r * 3 + 2]);
+          if (dZ > win) continue;
+          const double dist = sqrt(dX * dX + dY * dY + dZ * dZ);
+          if (dist < win) { win = dist; xi[0] = M.xGP[i]; xi[1] = M.xGP[j]; xi[2] = M.xGP[k]; }
+        }
+  } else {
+    xi[0] = xi[1] = xi[2] = 0.0;
   }
 }
 
