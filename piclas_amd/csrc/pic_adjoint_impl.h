@@ -658,13 +658,8 @@ int sc_push(pic_handle *h, double dt, const double *E) {
   const int32_t *nDev = h->start + h->hm.nElems;
   DevMesh M = h->M;
   M.E = E;
-  const dim3 grid(grid_for(std::max<int64_t>(n, 1)));
-  if (M.affine) { LAUNCH_N3(k_push_inside, h->hm.N, false, true, grid, M, h->P, n, dt, h->newElem, h->mv, nDev); }
-  else
-    LAUNCH_N(k_push_inside, h->hm.N, grid, M, h->P, n, dt, h->newElem, h->mv, nDev);
+  if (int rc = push_track(h, M, n, dt, nDev, false)) return rc;
   h->recFresh = false;
-  hipLaunchKernelGGL(k_track_movers<false>, dim3(mover_grid(n)), dim3(kBlock), 0, h->stream, h->M, h->P, h->newElem,
-                     h->mv, h->lostCount, h->insideById, h->stateById);
   HIPCHK(hipGetLastError());
   return enqueue_sort(h, n, false);
 }

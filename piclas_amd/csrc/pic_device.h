@@ -871,6 +871,13 @@ __device__ inline double intersection_with_wall(const DevMesh &M, int e, int l, 
   return alpha;
 }
 
+// On a parallelepiped: x is in element e, further than rounding from its faces
+__device__ inline bool inside_affine(const DevMesh &M, int e, const double x[3]) {
+  double xi[3];
+  affine_xi(M, e, x, xi);
+  return fmax(fabs(xi[0]), fmax(fabs(xi[1]), fabs(xi[2]))) < 1.0 - 1e-10;
+}
+
 // SingleParticleTriaTracking3D, particles/tracking/particle_triatracking.f90:137-484
 // (regular sides; open and periodic particle boundaries, particle_boundary_condition.f90:35-284).
 // x and last are updated in place by periodic shifts.  Returns the new owner
@@ -887,6 +894,8 @@ __device__ inline int tria_track(const DevMesh &M, int elem, double x[3], double
   steps = 0;
   for (int guard = 0; guard < 4096; ++guard) {
     ++steps;
+    // (in the elements the walk comes to on affine meshes xi mostly decides)
+    if (guard > 0 && M.affine && inside_affine(M, elem, x)) return elem;
     double det[6][2];
     if (inside_quad(M, elem, x, det)) return elem;
     traj[0] = x[0] - last[0];
