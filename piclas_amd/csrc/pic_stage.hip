@@ -432,13 +432,23 @@ __global__ __launch_bounds__(kBlock) void k_rm_movers(DevMesh M, DevParts P, int
 
 // Kernel C for RefMapping: ParticleBCTracking for the movers whose step may
 // hit a boundary side, and the search's fallback, from the state kernel A
-// left (the candidate bit holds the outcome of bc_may_hit)
+// left (the candidate bit holds the outcome of bc_may_hit).  324 registers and
+// 5 KB of stack per lane: one wave per SIMD, and a time that is the longest
+// chain of clips and Newton iterations in a wave.  So the list is dealt to as
+// many waves as are resident at once, a few lanes each where it is short: 256
+// workgroups 480 us for 6 million particles, full waves of 1024 workgroups
+// 830, spread over 1024 or 4096 workgroups 840 and 1130 (their stacks come
+// through the caches in turns); of 24 million 580 for 940, of 100,000 560 for 710.
+constexpr int kBcGroups = 256;
 template <int N, int G>
 __global__ __launch_bounds__(kBlock) void k_rm_bc_movers(DevMesh M, DevParts P, int32_t *newElem, Movers mv,
                                                          unsigned long long *lostCount, uint8_t *insideById,
                                                          double *stateById) {
   const int cnt = mv.count[kMoverSegs * kMoverLine];
-  for (int j = blockIdx.x * kBlock + threadIdx.x; j < cnt; j += gridDim.x * kBlock) {
+  const int waves = gridDim.x * (kBlock / kWave), lane = lane_id();
+  const int per = min((cnt + waves - 1) / waves, kWave);
+  if (lane >= per) return;
+  for (int j = (blockIdx.x * kBlock + threadIdx.x) / kWave * per + lane; j < cnt; j += waves * per) {
     const int i = mv.late[j];
     const int f = newElem[i];
     double x[3] = {P.x[i], P.y[i], P.z[i]};
@@ -3012,7 +3022,7 @@ int enqueue_step(pic_handle *h, double dt, int64_t nGrid, bool timed) {
     LAUNCH_NG(k_rm_movers, h->hm.N, h->hm.NGeo, moverGrid, h->M, h->P, h->newElem, h->mv, h->lostCount,
               h->insideById, h->stateById);
     if (h->hm.nBC > 0)
-      LAUNCH_NG(k_rm_bc_movers, h->hm.N, h->hm.NGeo, dim3(1024), h->M, h->P, h->newElem, h->mv, h->lostCount,
+      LAUNCH_NG(k_rm_bc_movers, h->hm.N, h->hm.NGeo, dim3(kBcGroups), h->M, h->P, h->newElem, h->mv, h->lostCount,
                 h->insideById, h->stateById);
   } else {
     if (int rc = push_track(h, h->M, nGrid, dt, nDev, timed)) return rc;
