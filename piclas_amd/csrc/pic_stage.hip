@@ -434,21 +434,25 @@ __global__ __launch_bounds__(kBlock) void k_rm_movers(DevMesh M, DevParts P, int
 // hit a boundary side, and the search's fallback, from the state kernel A
 // left (the candidate bit holds the outcome of bc_may_hit).  324 registers and
 // 5 KB of stack per lane: one wave per SIMD, and a time that is the longest
-// chain of clips and Newton iterations in a wave.  So the list is dealt to as
-// many waves as are resident at once, a few lanes each where it is short: 256
-// workgroups 480 us for 6 million particles, full waves of 1024 workgroups
-// 830, spread over 1024 or 4096 workgroups 840 and 1130 (their stacks come
-// through the caches in turns); of 24 million 580 for 940, of 100,000 560 for 710.
-constexpr int kBcGroups = 256;
+// chain of clips and Newton iterations in a wave.  So a list that the resident
+// waves can take at once is dealt to them, a few lanes each where it is short
+// (kBcResident workgroups): 480 us for 6 million particles, full waves 830,
+// spread over all 1024 or 4096 workgroups 840 and 1130 (their stacks come
+// through the caches in turns); of 24 million 580 for 940, of 100,000 560 for
+// 710.  A longer list goes to all workgroups in full waves (of 30 million that
+// reach further in a step 1150 us, by the resident waves alone 1390).
+constexpr int kBcGroups = 1024, kBcResident = 256;
 template <int N, int G>
 __global__ __launch_bounds__(kBlock) void k_rm_bc_movers(DevMesh M, DevParts P, int32_t *newElem, Movers mv,
                                                          unsigned long long *lostCount, uint8_t *insideById,
                                                          double *stateById) {
   const int cnt = mv.count[kMoverSegs * kMoverLine];
-  const int waves = gridDim.x * (kBlock / kWave), lane = lane_id();
-  const int per = min((cnt + waves - 1) / waves, kWave);
-  if (lane >= per) return;
-  for (int j = (blockIdx.x * kBlock + threadIdx.x) / kWave * per + lane; j < cnt; j += waves * per) {
+  const int resident = kBcResident * (kBlock / kWave), lane = lane_id();
+  const int waves = cnt <= resident * kWave ? resident : kBcGroups * (kBlock / kWave);
+  const int per = waves == resident ? (cnt + waves - 1) / waves : kWave;
+  const int w = (blockIdx.x * kBlock + threadIdx.x) / kWave;
+  if (w >= waves || lane >= per) return;
+  for (int j = w * per + lane; j < cnt; j += waves * per) {
     const int i = mv.late[j];
     const int f = newElem[i];
     double x[3] = {P.x[i], P.y[i], P.z[i]};
