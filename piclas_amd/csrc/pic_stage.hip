@@ -710,20 +710,25 @@ __global__ __launch_bounds__(kBlock) void k_dest(int64_t n, int nElems, const in
   else arr[s + stayCnt[ne] + ~r] = int32_t(i);
 }
 
-// The arrivals of an element in the order of their caller ids: 8 lanes per
+// The arrivals of an element in the order of their caller ids: LANES lanes per
 // element, each counting for its arrivals the smaller ids (an insertion sort
-// by one thread took 36 us where some tens arrive per element, now 11).
-constexpr int kFixLanes = 8;
+// by one thread took 36 us where some tens arrive per element, 8 lanes 11).  A
+// whole wave where the elements are few, as then it is the count of arrivals in
+// one that takes the time: 4,096 elements with a hundred or more each 111 -> 17
+// us, 8,000 with few 5 us either way, but 110,592 with few 15 us by 8 lanes and
+// 46 by 64.
+constexpr int kFixWaveElems = 8192;
 constexpr int64_t kFixInGather = int64_t(1) << 20;   // particles up to which k_gather_state does it
+template <int LANES>
 __global__ __launch_bounds__(kBlock) void k_fix_arrivals(int nElems, const int32_t *newStart, const int32_t *stayCnt,
                                                          const int32_t *arrCnt, const int32_t *id, const int32_t *arr,
                                                          int32_t *perm) {
-  const int t = blockIdx.x * kBlock + threadIdx.x, e = t / kFixLanes;
+  const int t = blockIdx.x * kBlock + threadIdx.x, e = t / LANES;
   if (e >= nElems) return;
   const int na = arrCnt[e];
   if (na == 0) return;
   const int b = newStart[e] + stayCnt[e];
-  for (int a = t % kFixLanes; a < na; a += kFixLanes) {
+  for (int a = t % LANES; a < na; a += LANES) {
     const int32_t v = arr[b + a], key = id[v];
     int r = 0;
     for (int k = 0; k < na; ++k) r += id[arr[b + k]] < key;
@@ -2449,7 +2454,8 @@ int enqueue_sort(pic_handle *h, int64_t nGrid, bool withStaged) {
   hipLaunchKernelGGL(scan ? k_dest<true> : k_dest<false>, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, n, ne,
                      h->newElem, h->rank, h->startNew, h->stayCnt, h->arrCnt, h->perm, fix ? h->perm : h->arr, nOld);
   if (!fix)
-    hipLaunchKernelGGL(k_fix_arrivals, dim3(grid_for(int64_t(ne) * kFixLanes)), dim3(kBlock), 0, h->stream, ne,
+    hipLaunchKernelGGL(ne <= kFixWaveElems ? k_fix_arrivals<kWave> : k_fix_arrivals<8>,
+                       dim3(grid_for(int64_t(ne) * (ne <= kFixWaveElems ? kWave : 8))), dim3(kBlock), 0, h->stream, ne,
                        h->startNew, h->stayCnt, h->arrCnt, h->P.id, h->arr, h->perm);
   const int32_t *total = h->startNew + ne;
   SpeciesFactor sfac{};

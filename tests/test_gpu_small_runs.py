@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from piclas_amd import mesh as M, stage, workloads as W
-from test_gpu_parity import run_pair
+from test_gpu_parity import deformed_box, run_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +43,24 @@ def test_walk_and_scan(oracle_mod, shape, N, n, graph):
     assert np.array_equal(s.part_source(), t.part_source())
     s.close()
     t.close()
+
+
+@pytest.mark.parametrize("nx", [3, 5, 21])
+def test_arrivals_in_caller_order(oracle_mod, nx):
+    """Many arrivals per element on general elements, where a wave (up to 8,192 elements) or 8 lanes order them:
+    the same bits in every run, though the atomics hand out the places in any order."""
+    n = max(40000, 8 * nx ** 3)
+    w = deformed_box(W.thermal_cube(nx=nx, ppc=-(-n // nx ** 3), steps=2))
+    out = []
+    for _ in range(3):
+        with stage.PICStage(w.mesh, w.N, max_particles=len(w.PartState), **W.stage_kwargs(w)) as s:
+            s.set_field(0.0 * w.E)
+            s.set_particles(w.PartState, elem=w.elem, species=w.species)
+            before = s.particles()[1]
+            s.time_step(3000 * w.dt, 2)   # a thermal step of 0.2
+            s.deposition()
+            out.append(s.particles() + (s.part_source(),))
+    assert (out[0][1] != before).sum() > len(before) // 4
+    for o in out[1:]:
+        for a, b in zip(out[0], o):
+            assert np.array_equal(a, b)
