@@ -2879,8 +2879,9 @@ int set_particles_impl(pic_handle *h, int64_t n, const double *PartState, const 
   // stable sort by element: the caller's order within one
   const int tiles = int(std::max<int64_t>(1, (n + kRadixTile - 1) / kRadixTile));
   const int32_t *key = h->newElem, *idx = nullptr;
-  for (int bit = 0; bit == 0 || (ne >> bit) > 0; bit += 8) {
-    int32_t *keyOut = (bit / 8) % 2 == 0 ? h->rank : h->Q.elem, *idxOut = (bit / 8) % 2 == 0 ? h->arr : h->Q.id;
+  for (int pass = 0; pass < radix_passes(ne); ++pass) {
+    const int bit = 8 * pass;
+    int32_t *keyOut = pass % 2 == 0 ? h->rank : h->Q.elem, *idxOut = pass % 2 == 0 ? h->arr : h->Q.id;
     hipLaunchKernelGGL(k_radix_count, dim3(tiles), dim3(kBlock), 0, h->stream, n, ne, key, bit, h->radixCnt);
     hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, h->stream, kRadixBins * tiles, h->radixCnt,
                        static_cast<const int32_t *>(nullptr), h->radixOff);

@@ -21,6 +21,14 @@ constexpr int kMaxNGeo = 2;       // geometry degree (TriaTracking: 1; RefMappin
 constexpr int kMaxSpecies = 8;
 constexpr int kMaxBinElems = 256;  // elements per RefMapping background cell
 
+// Passes of 8 bits that order the keys 0..nElems (nElems: a particle without
+// an element).  Never a fifth: a shift by the width of the type is undefined.
+constexpr int radix_passes(int32_t nElems) {
+  int p = 1;
+  while (p < 4 && (nElems >> (8 * p)) > 0) ++p;
+  return p;
+}
+
 // Host-side mesh tables: the reference's particle-mesh arrays, derived from
 // the HOPR arrays exactly as its init routines derive them.
 struct HostMesh {
