@@ -256,9 +256,9 @@ int  pic_adjoint(pic_handle *h, double dt, int32_t K, int32_t checkpoint_every, 
  *              that one wave takes a target element, the shape-function sums
  *              run as persistent waves, as many as the device holds at once,
  *              that take target elements from atomic counters (one per XCD
- *              range of elements).  Elsewhere the waves of a workgroup share
- *              a target, and this changes nothing.  Each target is summed in
- *              the same order, so the result is bit-identical.
+ *              range of elements).  Elsewhere this changes nothing.  Each
+ *              target is summed in the same order, so the result is
+ *              bit-identical.
  *   sf_shared_loads  1: on meshes that are not axis-aligned tensor grids, the
  *              four waves that share a target read every record of its source
  *              lists, without skipping the blocks of records whose bounding

@@ -1303,21 +1303,21 @@ __device__ inline int sf_next_target(const SFArgs &A, int nE, int &range, int la
 // are appended, and groups of 4 are consumed once 64 are pending, so groups
 // span source chunks and only the very last group is padded.
 // A target is up to 64 DOFs of an element: all of them for N <= 3 (in NQ
-// quarters of 16), one of its chunks of 64 for higher N.  The waves of a
-// workgroup share the target: wave wib takes every fourth source run, and
-// their sums are added in wave order.
+// quarters of 16), one of its chunks of 64 for higher N.  NW waves share the
+// target: wave wib takes every NW-th source run, and their sums are added in
+// wave order.
 constexpr int kRingMfma = 128;
 template <int N> struct GatherShape {
   static constexpr int nd = (N + 1) * (N + 1) * (N + 1), nch = (nd + kWave - 1) / kWave;
   static constexpr int NQ = nd >= 48 ? 4 : (nd + 15) / 16;
 };
-template <int N, int ALPHA, bool LINEAR>
+template <int N, int ALPHA, bool LINEAR, int NW>
 __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(const DevMesh &M, const int32_t *start,
                                                                             const SFArgs &A, double *PS, int tt,
                                                                             double (*L)[8], int lane, int wib) {
 #pragma clang fp contract(fast)
   constexpr int nd = GatherShape<N>::nd, nch = GatherShape<N>::nch, NQ = GatherShape<N>::NQ;
-  constexpr int kRing = kRingMfma, NW = kBlock / kWave;
+  constexpr int kRing = kRingMfma;
   const int t = nch == 1 ? tt : tt / nch, d0 = nch == 1 ? 0 : (tt % nch) * kWave;
   const double bx = M.bary[t * 3], by = M.bary[t * 3 + 1], bz = M.bary[t * 3 + 2];
   const double R2i0 = A.r2_sf_inv;
@@ -1377,7 +1377,7 @@ __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(cons
       ms0 = start[A.rfirst[qb + lane]]; ms1 = start[A.rend[qb + lane]]; msi = A.rshift[qb + lane];
     }
     const int jn = min(kWave, qend - qb);
-    for (int j = wib; j < jn; j += NW) {
+    for (int j = NW > 1 ? wib : 0; j < jn; j += NW) {
       const int s0 = __builtin_amdgcn_readlane(ms0, j), s1 = __builtin_amdgcn_readlane(ms1, j);
       const int si = __builtin_amdgcn_readlane(msi, j);
       // shifted position (GetPartPosShifted) relative to the target barycentre
@@ -1482,6 +1482,14 @@ __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(cons
     for (int g = 0; g < ng; ++g) group(L + (head & (kRing - 1)), g);
   }
   const int dofLo = 4 * ((lane >> 2) & 3) + (lane >> 4);
+  if (NW == 1) {
+#pragma unroll
+    for (int Q = 0; Q < NQ; ++Q) {
+      const int d = d0 + 16 * Q + dofLo;
+      if (nd % 64 == 0 || d < nd) PS[((size_t)t * nd + d) * 4 + jc] = acc[Q];
+    }
+    return;
+  }
   // the rings are done with: they hold the waves' sums
   double *part = &L[0][0];
   __builtin_amdgcn_wave_barrier();
@@ -1498,21 +1506,23 @@ __device__ __attribute__((always_inline)) inline void sf_gather_mfma_target(cons
   }
 }
 
-// One target per workgroup, its source runs dealt to the four waves.  With a
-// wave per target the wave of the fullest target ends long after the others
-// on a mesh with uneven occupancy (16 x 64 x 16 annulus, 6 million particles,
-// density e-folding over a tenth of the radius: 5.26 ms, now 3.05; 24 x 96 x
-// 24, 30 million: 15.8 ms, 14.8 as persistent waves, now 13.9), and small
-// meshes leave the device idle (1,000 deformed elements of 200: 335 us, now
-// 247).  Evenly filled large meshes take the same either way (27,000 of 111:
-// 2.69 ms); 16 waves per target are slower everywhere (4.2 and 20.8 ms).
-template <int N, int ALPHA, bool LINEAR>
+// NW = 4: one target per workgroup, its source runs dealt to the four waves.
+// With a wave per target the wave of the fullest target ends long after the
+// others on a mesh with uneven occupancy (16 x 64 x 16 annulus, 6 million
+// particles, density e-folding over a tenth of the radius: 5.26 ms, now 3.05;
+// 24 x 96 x 24, 30 million: 15.8 ms, 14.8 as persistent waves, now 13.9), and
+// small meshes leave the device idle (1,000 deformed elements of 200: 335 us,
+// now 247).  Evenly filled large meshes take the same either way (27,000 of
+// 111: 2.69 ms); 16 waves per target are slower everywhere (4.2 and 20.8 ms).
+// NW = 1: a target per wave, where a target has too few runs for four waves
+// (share_target).
+template <int N, int ALPHA, bool LINEAR, int NW>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_MX))) void k_sf_gather_mfma(DevMesh M, const int32_t *start, SFArgs A, double *PS) {
   __shared__ double lds[kBlock / kWave][kRingMfma][8];
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int t = xcd_block(blockIdx.x, gridDim.x);
+  const int b = xcd_block(blockIdx.x, gridDim.x), t = NW == 1 ? b * (kBlock / kWave) + wib : b;
   if (t < M.nElems * GatherShape<N>::nch)
-    sf_gather_mfma_target<N, ALPHA, LINEAR>(M, start, A, PS, t, lds[wib], lane_id(), wib);
+    sf_gather_mfma_target<N, ALPHA, LINEAR, NW>(M, start, A, PS, t, lds[wib], lane_id(), NW == 1 ? 0 : wib);
 }
 
 // The same gather for targets whose Gauss points form an axis-aligned tensor
@@ -2143,6 +2153,7 @@ struct pic_handle {
   bool sfMatrix = true;   // N = 3 shape function: accumulate on the matrix cores
   bool recFresh = false;  // sf.rec holds the records of the current particle arrays
   bool useGraph = false;  // replay captured two-step graphs in pic_time_step
+  int32_t sfRuns = 0;     // runs of source elements of all targets
   bool sfPersist = false; // N = 3 matrix-core gathers: persistent waves that take targets from counters
   bool sfNoSkip = false;  // general matrix-core gather: no record block is skipped
   int nCU = 0;            // compute units of the device
@@ -2296,6 +2307,21 @@ int emit_scratch_init(int device);
 int set_particles_impl(pic_handle *h, int64_t n, const double *PartState, const int32_t *elem, const int32_t *species,
                        const uint8_t *is_new, bool outsideMarked);
 
+// Whether nw waves share a target.  They take its runs of source elements in
+// turn, and a wave without a run keeps others out, unless all waves of the
+// launch are resident together anyway (4,096 are).  A mesh one element thick
+// in two directions has one run per target, in one direction three to five
+// (and a few from periodic shifts), any other nine or more, fewer at walls.
+// Us with one wave / four: 27,000 deformed elements in a row of 100 particles
+// 271 / 485; 160 x 160 x 1 of 100, three runs 320 / 410, five 837 / 890; on a
+// tensor grid 4,000 in a row 87 / 147, 120 x 120 x 1 of 200 804 / 835.  With
+// nine runs (30^3 deformed elements of 100) 690 / 765, but unevenly filled
+// meshes of nine need the four (k_sf_gather_mfma).  Eight waves: 2,000 in a
+// row 47 / 126; with 25 runs they gain.
+bool share_target(const pic_handle *h, int64_t targets, int nw) {
+  return targets * nw <= 4096 || int64_t(h->sfRuns) * 8 > int64_t(h->hm.nElems) * 11 * nw;   // 1.375 runs a wave
+}
+
 // Waves that share a target of the tensor-grid gather.  One wave per target
 // leaves the device idle below some 10^4 elements (4,096 waves are resident):
 // a step's gather took, in us with 1 / 4 / 8 / 16 waves per target, 1,000
@@ -2308,8 +2334,8 @@ int set_particles_impl(pic_handle *h, int64_t n, const double *PartState, const 
 int gather_waves(const pic_handle *h) {
   const int64_t ne = h->hm.nElems;
   if (ne <= 256) return 16;
-  if (ne <= 2048) return 8;
-  if (ne <= 4096 || (ne <= 16384 && h->nTotal >= 64 * ne)) return 4;
+  if (ne <= 2048 && share_target(h, ne, 8)) return 8;
+  if ((ne <= 4096 || (ne <= 16384 && h->nTotal >= 64 * ne)) && share_target(h, ne, 4)) return 4;
   return 1;
 }
 
@@ -2398,12 +2424,19 @@ int run_deposition(pic_handle *h, bool timed) {
         else SF_CART(0);
 #undef SF_CART
       } else {
-        const unsigned grid = xcd_grid(int64_t(ne) * ((h->hm.nDof + kWave - 1) / kWave));
-#define SF_GENERAL(N, LIN)                                                       \
-  do {                                                                          \
-    if (a.alpha == 2) SF_LAUNCH((k_sf_gather_mfma<N, 2, LIN>), grid, kBlock);    \
-    else if (a.alpha == 3) SF_LAUNCH((k_sf_gather_mfma<N, 3, LIN>), grid, kBlock); \
-    else SF_LAUNCH((k_sf_gather_mfma<N, 0, LIN>), grid, kBlock);                 \
+        const int64_t targets = int64_t(ne) * ((h->hm.nDof + kWave - 1) / kWave);
+        const bool share = share_target(h, targets, waves);
+        const unsigned grid = xcd_grid(share ? targets : (targets + waves - 1) / waves);
+#define SF_GENERAL_NW(N, LIN, NW)                                                      \
+  do {                                                                                \
+    if (a.alpha == 2) SF_LAUNCH((k_sf_gather_mfma<N, 2, LIN, NW>), grid, kBlock);      \
+    else if (a.alpha == 3) SF_LAUNCH((k_sf_gather_mfma<N, 3, LIN, NW>), grid, kBlock); \
+    else SF_LAUNCH((k_sf_gather_mfma<N, 0, LIN, NW>), grid, kBlock);                   \
+  } while (0)
+#define SF_GENERAL(N, LIN)                          \
+  do {                                             \
+    if (share) SF_GENERAL_NW(N, LIN, kBlock / kWave); \
+    else SF_GENERAL_NW(N, LIN, 1);                  \
   } while (0)
         switch (N) {
           case 1: SF_GENERAL(1, false); break;
@@ -2419,6 +2452,7 @@ int run_deposition(pic_handle *h, bool timed) {
           default: break;
         }
 #undef SF_GENERAL
+#undef SF_GENERAL_NW
       }
 #undef SF_LAUNCH
     } else if (h->sf.alpha == 2) {
@@ -2691,6 +2725,7 @@ int pic_create(const pic_mesh_desc *mesh, const pic_params *par, pic_handle **ou
     rc |= upload(h, const_cast<int32_t **>(&h->sf.src), hm.sfSrc);
     rc |= upload(h, const_cast<uint8_t **>(&h->sf.shift), hm.sfShift);
     rc |= upload(h, const_cast<int32_t **>(&h->sf.roff), hm.sfRunOff);
+    h->sfRuns = hm.sfRunOff.back();
     rc |= upload(h, const_cast<int32_t **>(&h->sf.rfirst), hm.sfRunFirst);
     rc |= upload(h, const_cast<int32_t **>(&h->sf.rend), hm.sfRunEnd);
     rc |= upload(h, const_cast<uint8_t **>(&h->sf.rshift), hm.sfRunShift);
