@@ -239,7 +239,14 @@ int  pic_field_energy(pic_handle *h, double *WEl);
  *                     with respect to the positions and velocities at entry
  *                     (caller order, [nPart][3]); the states are recomputed
  *                     from checkpoints every checkpoint_every steps.  Leaves the
- *                     stage in the state after K steps. */
+ *                     stage in the state after K steps.  The handle holds until
+ *                     pic_destroy: K / checkpoint_every + checkpoint_every
+ *                     particle states, and for gradients the fields of the K
+ *                     steps, unless these exceed 16 GiB
+ *                     (PIC_ADJOINT_FIELD_BYTES in the environment sets another
+ *                     limit), half of the free memory, or cannot be allocated:
+ *                     then the fields of checkpoint_every steps, which are
+ *                     deposited a second time. */
 int  pic_set_field_operator(pic_handle *h, const double *G);
 int  pic_sc_time_step(pic_handle *h, double dt, int32_t nsteps, double *loss);
 int  pic_adjoint(pic_handle *h, double dt, int32_t K, int32_t checkpoint_every, double *loss, double *dLdx0,

@@ -577,17 +577,84 @@ __global__ void k_copy_f64(const double *a, double *b, int64_t n) {
 }
 
 // ---- host side ------------------------------------------------------------------
-constexpr size_t kFieldBytes = size_t(16) << 30;   // most memory for the fields of the forward steps
+// most memory for the fields of the forward steps
+constexpr size_t kFieldBytes = size_t(16) << 30;
 
-int alloc_state(pic_handle *h, StepState &S, bool withE) {
+// device memory that the call can do without: null where there is none
+double *try_alloc(pic_handle *h, size_t count) {
+  void *q = nullptr;
+  if (hipMalloc(&q, count * sizeof(double)) != hipSuccess) {
+    (void)hipGetLastError();   // (not left for the next check)
+    return nullptr;
+  }
+  h->allocs.push_back(q);
+  return static_cast<double *>(q);
+}
+template <typename T>
+void release(pic_handle *h, T *&p) {
+  if (!p) return;
+  h->allocs.erase(std::find(h->allocs.begin(), h->allocs.end(), static_cast<void *>(p)));
+  (void)hipFree(p);
+  p = nullptr;
+}
+void release_fields(pic_handle *h) {
+  for (double *&E : h->adj.Es) release(h, E);
+  h->adj.Es.clear();
+}
+
+int alloc_state(pic_handle *h, StepState &S) {
   int rc = 0;
   rc |= dalloc(h, &S.x, size_t(h->cap) * 6);
   rc |= dalloc(h, &S.elem, h->cap);
   rc |= dalloc(h, &S.id, h->cap);
   rc |= dalloc(h, &S.spec, h->cap);
   rc |= dalloc(h, &S.start, h->hm.nElems + 1);
-  if (withE) rc |= dalloc(h, &S.E, size_t(h->hm.nElems) * h->hm.nDof * 3);
+  if (rc) {   // all or nothing: a later call tries again
+    (void)hipGetLastError();
+    release(h, S.x); release(h, S.elem); release(h, S.id); release(h, S.spec); release(h, S.start);
+  }
   return rc;
+}
+
+// What every call of pic_adjoint needs: the checkpoints, and for gradients
+// the states of one segment (the first one's slot holds the state after the
+// last step) and the adjoint vectors.
+int alloc_required(pic_handle *h, int nck, int every, bool backward) {
+  Adjoint &a = h->adj;
+  if (int(a.ck.size()) < nck) a.ck.resize(nck);
+  for (int c = 0; c < nck; ++c)
+    if (!a.ck[c].x && alloc_state(h, a.ck[c])) return PIC_EHIP;
+  if (!backward) return 0;
+  if (int(a.seg.size()) < every) a.seg.resize(every);
+  for (int c = 0; c < every; ++c)
+    if (!a.seg[c].x && alloc_state(h, a.seg[c])) return PIC_EHIP;
+  for (double **v : {&a.lx, &a.lv, &a.lF, &a.xi})
+    if (!*v && dalloc(h, v, size_t(h->cap) * 3)) {
+      (void)hipGetLastError();
+      return PIC_EHIP;
+    }
+  return 0;
+}
+
+// The fields of K steps of nE3 values, if they fit kFieldBytes (or
+// PIC_ADJOINT_FIELD_BYTES) and half of the memory that is free, and the
+// allocations succeed; else none are held.
+bool keep_fields(pic_handle *h, int K, size_t nE3) {
+  std::vector<double *> &Es = h->adj.Es;
+  if (int(Es.size()) >= K) return true;
+  size_t limit = kFieldBytes, avail = 0, total = 0;
+  if (const char *k = std::getenv("PIC_ADJOINT_FIELD_BYTES")) limit = std::strtoull(k, nullptr, 10);
+  const size_t bytes = nE3 * sizeof(double);
+  if (hipMemGetInfo(&avail, &total) == hipSuccess) limit = std::min(limit, Es.size() * bytes + avail / 2);
+  while (int(Es.size()) < K) {
+    double *E = (Es.size() + 1) * bytes <= limit ? try_alloc(h, nE3) : nullptr;
+    if (!E) {
+      release_fields(h);
+      return false;
+    }
+    Es.push_back(E);
+  }
+  return true;
 }
 
 void copy_state(pic_handle *h, const StateCopy &C, int64_t n) {
@@ -765,45 +832,31 @@ int pic_adjoint(pic_handle *h, double dt, int32_t K, int32_t every, double *loss
   if (set_device(h)) return PIC_EHIP;
   Adjoint &a = h->adj;
   const int nck = (K + every - 1) / every;
-  // buffers: checkpoints, one segment of step states, adjoint vectors
-  if (int(a.ck.size()) < nck) {
-    a.ck.resize(nck);
-    for (int c = 0; c < nck; ++c)
-      if (!a.ck[c].x && alloc_state(h, a.ck[c], false)) return PIC_EHIP;
+  const bool backward = dLdx0 || dLdv0;
+  const int64_t nE3 = int64_t(h->hm.nElems) * h->hm.nDof * 3;
+  if (alloc_required(h, nck, every, backward)) {
+    release_fields(h);   // (of an earlier call)
+    if (int rc = alloc_required(h, nck, every, backward)) return rc;
   }
-  if (int(a.seg.size()) < every) {
-    a.seg.resize(every);
+  // The field of every forward step is kept where there is room, so that the
+  // reverse sweep recomputes positions and velocities only (a deposition
+  // costs some ten pushes); else it keeps those of a segment and deposits
+  // again, and runs the last steps again at the end.
+  const bool keep = backward && keep_fields(h, K, size_t(nE3));
+  if (backward && !keep)
     for (int c = 0; c < every; ++c)
-      if (!a.seg[c].x && alloc_state(h, a.seg[c], true)) return PIC_EHIP;
-  }
-  if (!a.lx) {
-    int rc = 0;
-    rc |= dalloc(h, &a.lx, size_t(h->cap) * 3);
-    rc |= dalloc(h, &a.lv, size_t(h->cap) * 3);
-    rc |= dalloc(h, &a.lF, size_t(h->cap) * 3);
-    rc |= dalloc(h, &a.xi, size_t(h->cap) * 3);
-    if (rc) return PIC_EHIP;
-  }
+      if (!a.seg[c].E && !(a.seg[c].E = try_alloc(h, nE3)))
+        return fail(PIC_EHIP, "pic_adjoint: no device memory for the fields of a segment");
+  // what the stage holds after K steps; without room, the last ones are run again
+  if (keep && !a.finE) a.finE = try_alloc(h, nE3);
+  if (keep && !a.PS) a.PS = try_alloc(h, nE3 / 3 * 4);
+  const bool fin = keep && a.finE && a.PS;
   const int64_t n = h->n;
   // the steps start from running particles (no IsNewPart half step)
   hipLaunchKernelGGL(k_fill_u8, dim3(grid_for(std::max<int64_t>(n, 1))), dim3(kBlock), 0, h->stream, h->P.isNew, n,
                      uint8_t(0));
   const int N = h->hm.N;
   const int ne = h->hm.nElems;
-  const int64_t nE3 = int64_t(ne) * h->hm.nDof * 3;
-  const bool backward = dLdx0 || dLdv0;
-  // The field of every forward step is kept, so that the reverse sweep
-  // recomputes positions and velocities only (a deposition costs some ten
-  // pushes); beyond kFieldBytes it keeps none and deposits again.
-  const bool keep = backward && size_t(K) * nE3 * sizeof(double) <= kFieldBytes;
-  for (int it = int(a.Es.size()); keep && it < K; ++it) {
-    double *E = nullptr;
-    if (dalloc(h, &E, nE3)) return PIC_EHIP;
-    a.Es.push_back(E);
-  }
-  if (backward && !a.fin.x) {
-    if (alloc_state(h, a.fin, true) || dalloc(h, &a.PS, size_t(ne) * h->hm.nDof * 4)) return PIC_EHIP;
-  }
   auto copy = [&](const double *src, double *dst, int64_t cnt) {
     hipLaunchKernelGGL(k_copy_f64, dim3(grid_for(cnt)), dim3(kBlock), 0, h->stream, src, dst, cnt);
   };
@@ -813,9 +866,9 @@ int pic_adjoint(pic_handle *h, double dt, int32_t K, int32_t every, double *loss
       if (int rc = save_state(h, a.ck[it / every])) return rc;
     if (int rc = sc_step(h, dt, keep ? a.Es[it] : h->E)) return rc;
   }
-  if (backward) {   // what the stage holds after K steps
-    if (int rc = save_state(h, a.fin)) return rc;
-    copy(keep ? a.Es[K - 1] : h->E, a.fin.E, nE3);
+  if (fin) {
+    if (int rc = save_state(h, a.seg[0])) return rc;
+    copy(a.Es[K - 1], a.finE, nE3);
     copy(h->PS, a.PS, nE3 / 3 * 4);
   }
   if (int rc = sc_loss(h, loss)) return rc;
@@ -860,9 +913,14 @@ int pic_adjoint(pic_handle *h, double dt, int32_t K, int32_t every, double *loss
     }
   }
   // the stage ends in the state after K steps
-  if (int rc = restore_state(h, a.fin)) return rc;
-  copy(a.fin.E, h->E, nE3);
-  copy(a.PS, h->PS, nE3 / 3 * 4);
+  if (int rc = restore_state(h, fin ? a.seg[0] : a.ck[nck - 1])) return rc;
+  if (fin) {
+    copy(a.finE, h->E, nE3);
+    copy(a.PS, h->PS, nE3 / 3 * 4);
+  } else {
+    for (int it = (nck - 1) * every; it < K; ++it)
+      if (int rc = sc_step(h, dt, h->E)) return rc;
+  }
   HIPCHK(hipStreamSynchronize(h->stream));
   const int64_t nt = h->nTotal;
   if (dLdx0) HIPCHK(hipMemcpy(dLdx0, a.lx, nt * 3 * sizeof(double), hipMemcpyDeviceToHost));

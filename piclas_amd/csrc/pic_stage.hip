@@ -2113,7 +2113,7 @@ struct Adjoint {
   uint8_t *tgtShift = nullptr;
   std::vector<StepState> ck, seg;
   std::vector<double *> Es;   // fields of the forward steps
-  StepState fin;              // the state after the forward steps
+  double *finE = nullptr;     // with PS and the first of seg: the stage after the forward steps
 };
 }  // namespace
 
