@@ -371,14 +371,50 @@ __device__ inline double min_key(double a, double b) {
   return r;
 }
 
-// Guess 2 in a wave of one element: the Gauss point nearest to x.  The
-// reference visits the points with the third index fastest and keeps the
-// first of equally near ones.  Here they come in memory order, 16 values per
-// scalar load and wait, and the point's place in the reference's order stands
-// in the last bits of its squared distance, so that one minimum compares
-// both (distances that agree to 2^-43 or better count as equal).  A load and
-// wait per point, the square roots and the early exits had made the push of
-// 6 million particles on a curved mesh (degree 3) 1675 us; so it takes 1494.
+// the middle one of three
+__device__ inline uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t c) {
+  uint32_t r;
+  asm("v_med3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// Guess 2: the Gauss point nearest to x, the first of equally near ones in the
+// reference's order (the third index fastest)
+template <int N>
+__device__ inline void nearest_gauss_point(const DevMesh &M, int e, const double x[3], double xi[3]) {
+  constexpr int n1 = N + 1;
+  const double *xg = M.xGPe + (size_t)e * n1 * n1 * n1 * 3;
+  const double d0[3] = {x[0] - xg[0], x[1] - xg[1], x[2] - xg[2]};
+  double win = sqrt(d0[0] * d0[0] + d0[1] * d0[1] + d0[2] * d0[2]);
+  xi[0] = xi[1] = xi[2] = M.xGP[0];
+#pragma unroll 1
+  for (int i = 0; i < n1; ++i)
+#pragma unroll 1
+    for (int j = 0; j < n1; ++j)
+#pragma unroll 1
+      for (int k = 0; k < n1; ++k) {
+        const int r = (k * n1 + j) * n1 + i;
+        const double dX = fabs(x[0] - xg[r * 3]);
+        if (dX > win) continue;
+        const double dY = fabs(x[1] - xg[r * 3 + 1]);
+        if (dY > win) continue;
+        const double dZ = fabs(x[2] - xg[r * 3 + 2]);
+        if (dZ > win) continue;
+        const double dist = sqrt(dX * dX + dY * dY + dZ * dZ);
+        if (dist < win) { win = dist; xi[0] = M.xGP[i]; xi[1] = M.xGP[j]; xi[2] = M.xGP[k]; }
+      }
+}
+
+// The same in a wave of one element.  The points come in memory order, 16
+// values per scalar load and wait, and the point's place in the reference's
+// order stands in the last bits of its squared distance, so that one minimum
+// finds both.  The upper words of the two smallest distances tell whether that
+// decides: where they are neighbours (one particle in some 10^5) the distances
+// may agree to the last bits, and the lane compares them as above, so that
+// a particle's start does not depend on its wave.  A load and wait per point,
+// the square roots and the early exits had made the push of 6 million
+// particles on a curved mesh (degree 3) 1675 us; so it takes 1484, and 1471
+// without the upper words.
 template <int N>
 __device__ inline void nearest_gauss_point_s(const DevMesh &M, int e, const double x[3], double xi[3]) {
   constexpr int n1 = N + 1, NP = n1 * n1 * 3;
@@ -386,6 +422,7 @@ __device__ inline void nearest_gauss_point_s(const DevMesh &M, int e, const doub
   constexpr uint32_t kMask = (1u << kBits) - 1;
   const double *xg = M.xGPe + (size_t)e * n1 * n1 * n1 * 3;
   double best = HUGE_VAL, d2 = 0.0;
+  uint32_t hi1 = ~0u, hi2 = ~0u;   // the smallest upper words (of a distance that is no number, one above all others)
 #pragma unroll 1
   for (int k = 0; k < n1; ++k) {
     double near = HUGE_VAL;
@@ -402,14 +439,20 @@ __device__ inline void nearest_gauss_point_s(const DevMesh &M, int e, const doub
           d2 = c == 0 ? d * d : __builtin_fma(d, d, d2);
           if (c == 2) {
             const uint64_t u = __builtin_bit_cast(uint64_t, d2);
-            const uint32_t lo = (uint32_t(u) & ~kMask) | uint32_t((i * n1 + j) * n1);
-            near = min_key(near, dw_to_d(lo, uint32_t(u >> 32)));
+            const uint32_t lo = (uint32_t(u) & ~kMask) | uint32_t((i * n1 + j) * n1), hi = uint32_t(u >> 32);
+            near = min_key(near, dw_to_d(lo, hi));
+            hi2 = med3_u32(hi1, hi2, hi);
+            hi1 = min(hi1, hi);
           }
         }
       }
     }
     const uint64_t u = __builtin_bit_cast(uint64_t, near);
     best = min_key(best, dw_to_d(uint32_t(u) + uint32_t(k), uint32_t(u >> 32)));
+  }
+  if (hi2 - hi1 <= 1u) {
+    nearest_gauss_point<N>(M, e, x, xi);
+    return;
   }
   const int at = int(uint32_t(__builtin_bit_cast(uint64_t, best)) & kMask);
   xi[0] = M.xGP[at / (n1 * n1)];
@@ -437,31 +480,8 @@ __device__ inline void ref_newton_start(const DevMesh &M, int e, const double x[
 #pragma unroll
       for (int d = 0; d < 3; ++d) xi[d] = fmax(fmin(1.0, xi[d]), -1.0);
   } else if (M.refGuess == 2) {
-    if (UNI) {
-      nearest_gauss_point_s<N>(M, e, x, xi);
-      return;
-    }
-    constexpr int n1 = N + 1;
-    const double *xg = M.xGPe + (size_t)e * n1 * n1 * n1 * 3;
-    const double d0[3] = {x[0] - xg[0], x[1] - xg[1], x[2] - xg[2]};
-    double win = sqrt(d0[0] * d0[0] + d0[1] * d0[1] + d0[2] * d0[2]);
-    xi[0] = xi[1] = xi[2] = M.xGP[0];
-#pragma unroll 1
-    for (int i = 0; i < n1; ++i)
-#pragma unroll 1
-      for (int j = 0; j < n1; ++j)
-#pragma unroll 1
-        for (int k = 0; k < n1; ++k) {
-          const int r = (k * n1 + j) * n1 + i;
-          const double dX = fabs(x[0] - xg[r * 3]);
-          if (dX > win) continue;
-          const double dY = fabs(x[1] - xg[r * 3 + 1]);
-          if (dY > win) continue;
-          const double dZ = fabs(x[2] - xg[r * 3 + 2]);
-          if (dZ > win) continue;
-          const double dist = sqrt(dX * dX + dY * dY + dZ * dZ);
-          if (dist < win) { win = dist; xi[0] = M.xGP[i]; xi[1] = M.xGP[j]; xi[2] = M.xGP[k]; }
-        }
+    if (UNI) nearest_gauss_point_s<N>(M, e, x, xi);
+    else nearest_gauss_point<N>(M, e, x, xi);
   } else {
     xi[0] = xi[1] = xi[2] = 0.0;
   }
