@@ -19,11 +19,14 @@ from . import workloads as W
 
 
 def candidates(N, deposition=stage.DEPO_SF):
+    """The variants of a stage of degree N: the shape-function kernel at every degree, persistent waves where the
+    tensor-grid kernel exists (N = 3)."""
     out = []
     for g in (False, True):
-        for k in ((1, 2) if N == 3 and deposition == stage.DEPO_SF else (0,)):
-            for p, c in (((False, False), (True, False), (False, True)) if k == 2 else ((False, False),)):
-                out.append({"use_graph": g, "sf_kernel": k, "sf_persistent": p, "sf_shared_loads": c})
+        for k in ((1, 2) if deposition == stage.DEPO_SF else (0,)):
+            for p, c in ((False, False), (True, False), (False, True)) if k == 2 else ((False, False),):
+                if not p or N == 3:
+                    out.append({"use_graph": g, "sf_kernel": k, "sf_persistent": p, "sf_shared_loads": c})
     return out
 
 
