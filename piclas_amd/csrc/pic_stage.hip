@@ -125,7 +125,6 @@ struct Movers {
   int32_t *idx;     // [kMoverSegs][seg] particles
   int64_t seg;      // places per segment
   int32_t *late;    // [cap] RefMapping: the particles that k_rm_movers passes on
-  double *last;     // [cap][3] positions of particles to be checked (restart)
 };
 // places per segment: all particles of the workgroups that share it
 inline int64_t mover_seg(int64_t cap) { return ((cap + kBlock - 1) / kBlock + kMoverSegs - 1) / kMoverSegs * kBlock; }
@@ -220,8 +219,8 @@ template <int N, bool MIXED = false, bool AFFINE = false, bool WALK = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE_PUSH))) void k_push_inside(DevMesh M, DevParts P, int64_t n, double dt, int32_t *newElem,
                                                         Movers mv, const int32_t *nDev, Removed rm = {}) {
   const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (nDev) n = *nDev;
-  bool mover = false;   // particle count on the device (graph replay)
+  if (nDev) n = *nDev;   // particle count on the device (graph replay)
+  bool mover = false;
   // whether all particles of the wave sit in one element (sorted order: most
   // waves); its field is then read by scalar loads
   const int eAll = i < n ? P.elem[i] : -1;
@@ -2816,7 +2815,6 @@ int pic_create(const pic_mesh_desc *mesh, const pic_params *par, pic_handle **ou
   rc |= dalloc(h, &h->mv.count, kMoverCounters);
   h->mv.seg = mover_seg(cap);
   rc |= dalloc(h, &h->mv.idx, size_t(h->mv.seg) * kMoverSegs);
-  rc |= dalloc(h, &h->mv.last, cap * 3);
   if (par->tracking == PIC_TRACK_REFMAPPING) {
     rc |= dalloc(h, &h->mv.late, cap);
   }

@@ -85,11 +85,12 @@ int pic_restart_particles(pic_handle *h, int64_t n, const double *PartData, cons
     std::vector<double> xyz(size_t(n) * 3);
     for (int64_t p = 0; p < n; ++p)
       for (int c = 0; c < 3; ++c) xyz[p * 3 + c] = state[p * 6 + c];
-    HIPCHK(copy_bytes(h->mv.last, xyz.data(), size_t(n) * 3 * sizeof(double), hipMemcpyHostToDevice));
+    double *pos = h->Q.F;   // scratch, as in set_particles_impl
+    HIPCHK(copy_bytes(pos, xyz.data(), size_t(n) * 3 * sizeof(double), hipMemcpyHostToDevice));
     HIPCHK(copy_bytes(h->newElem, el.data(), size_t(n) * sizeof(int32_t), hipMemcpyHostToDevice));
     const bool refmap = h->par.tracking == PIC_TRACK_REFMAPPING;
-    if (refmap) { LAUNCH_NG(k_rm_restart_check, h->hm.N, h->hm.NGeo, dim3(grid_for(n)), h->M, n, h->mv.last, h->newElem); }
-    else hipLaunchKernelGGL(k_tria_restart_check, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, h->M, n, h->mv.last,
+    if (refmap) { LAUNCH_NG(k_rm_restart_check, h->hm.N, h->hm.NGeo, dim3(grid_for(n)), h->M, n, pos, h->newElem); }
+    else hipLaunchKernelGGL(k_tria_restart_check, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, h->M, n, pos,
                             h->newElem);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -97,8 +98,8 @@ int pic_restart_particles(pic_handle *h, int64_t n, const double *PartData, cons
     HIPCHK(copy_bytes(chk.data(), h->newElem, size_t(n) * sizeof(int32_t), hipMemcpyDeviceToHost));
     for (int64_t p = 0; p < n; ++p) missing += chk[p] < 0;
     if (missing > 0) {
-      if (refmap) { LAUNCH_NG(k_rm_locate, h->hm.N, h->hm.NGeo, dim3(grid_for(n)), h->M, n, h->mv.last, 3, h->newElem); }
-      else hipLaunchKernelGGL(k_tria_locate, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, h->M, n, h->mv.last, 3,
+      if (refmap) { LAUNCH_NG(k_rm_locate, h->hm.N, h->hm.NGeo, dim3(grid_for(n)), h->M, n, pos, 3, h->newElem); }
+      else hipLaunchKernelGGL(k_tria_locate, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, h->M, n, pos, 3,
                               h->newElem);
       HIPCHK(hipGetLastError());
       HIPCHK(hipStreamSynchronize(h->stream));
