@@ -268,7 +268,7 @@ def main():
         stage.KERNEL_SF_CARTESIAN: ("k_sf_gather_cart<%d, false>" % a,
                                     "FP64 issue bound: per pair a subtraction, the clamp and the square on the VALU "
                                     "(axis-aligned tensor grid of Gauss points), products summed on FP64 MFMA (4x4x4)"),
-        stage.KERNEL_SF_MATRIX: ("k_sf_gather_mfma<%d, %d, true>" % (w.N, a),
+        stage.KERNEL_SF_MATRIX: ("k_sf_gather_mfma<%d, %d, %s, 4>" % (w.N, a, "true" if w.N == 3 else "false"),
                                  "FP64 issue bound: S on the VALU, its products summed on FP64 MFMA (4x4x4)"),
     }.get(st["deposit_kernel"], ("k_sf_gather<%d, %d>" % (w.N, 2 if a == 2 else 0), "FP64 issue bound: all on the VALU"))
     note += "; peak = MI355X FP64 vector peak (the FP64 matrix peak is the same 78.6 TFLOP/s)"
@@ -278,7 +278,7 @@ def main():
             "kernel": kname, "avg_launch_ms": round(avg_ms, 4),
             "algorithmic_flops_per_particle": round(fpp, 1), "note": note}
     ms_step = t / args.steps * 1e3
-    push = push_roofline(st, n_now, args.steps, "k_push_inside<3, false, true>", PUSH_BYTES_AFFINE,
+    push = push_roofline(st, n_now, args.steps, "k_push_inside<3, false, true, false>", PUSH_BYTES_AFFINE,
                          (args.nx ** 3) * 2208)
     if push is not None:
         push["traffic"] = measured_traffic(push["kernel"]) if (args.nx, args.ppc) == (48, 200) else None
