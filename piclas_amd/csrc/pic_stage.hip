@@ -2323,17 +2323,16 @@ int set_particles_impl(pic_handle *h, int64_t n, const double *PartState, const 
 
 // Whether nw waves share a target.  They take its runs of source elements in
 // turn, and a wave without a run keeps others out, unless all waves of the
-// launch are resident together anyway (4,096 are).  A mesh one element thick
-// in two directions has one run per target, in one direction three to five
-// (and a few from periodic shifts), any other nine or more, fewer at walls.
-// Us with one wave / four: 27,000 deformed elements in a row of 100 particles
-// 271 / 485; 160 x 160 x 1 of 100, three runs 320 / 410, five 837 / 890; on a
-// tensor grid 4,000 in a row 87 / 147, 120 x 120 x 1 of 200 804 / 835.  With
-// nine runs (30^3 deformed elements of 100) 690 / 765, but unevenly filled
-// meshes of nine need the four (k_sf_gather_mfma).  Eight waves: 2,000 in a
-// row 47 / 126; with 25 runs they gain.
+// launch are resident together anyway (4,096 are).  A row of elements has one
+// run per target, a sheet three to five, any other mesh nine or more.  Us with
+// one wave / four, rows: 27,000 deformed elements of 100 particles 275 / 500, on
+// a tensor grid 4,000 87 / 146 and 2,000 47 / 126 by eight.  Sheets: 160 x 160
+// x 1 deformed, three runs 330 / 420, but with the density falling off as the
+// root of x 490 / 460 and as its 3/4th power 900 / 630; 120 x 120 x 1 on a tensor
+// grid, five runs 800 / 860, 1183 / 918 and 1966 / 1080; 45 x 45 x 1, three runs
+// 60 by one, 64 by four, 92 by eight.  So waves share where most have a run.
 bool share_target(const pic_handle *h, int64_t targets, int nw) {
-  return targets * nw <= 4096 || int64_t(h->sfRuns) * 8 > int64_t(h->hm.nElems) * 11 * nw;   // 1.375 runs a wave
+  return targets * nw <= 4096 || int64_t(h->sfRuns) * 8 > int64_t(h->hm.nElems) * 5 * nw;   // 5/8 of a run each
 }
 
 // Waves that share a target of the tensor-grid gather.  One wave per target

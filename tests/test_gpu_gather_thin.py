@@ -1,7 +1,8 @@
-"""Shape-function deposition on meshes one element thick, whose targets have one
-to five runs of source elements: from 1,025 targets on a wave takes a target,
-below four or more share it.  Tensor grids, deformed and curved elements,
-degrees with one and with several chunks of 64 DOFs, against the oracle."""
+"""Shape-function deposition on rows and sheets of elements, whose targets have
+one and three to five runs of source elements: a wave takes a target of a row from
+1,025 targets on, four or more share it elsewhere.  Tensor grids, deformed and
+curved elements, degrees with one and with several chunks of 64 DOFs, against the
+oracle."""
 import numpy as np
 import pytest
 
@@ -17,8 +18,9 @@ pytestmark = pytest.mark.gpu
                                             ("box", (33, 32, 1), 5000, 3), ("box", (1026, 1, 1), 4000, 1),
                                             ("box", (1, 1030, 1), 2000, 4), ("box", (1, 1, 150), 700, 7),
                                             ("deformed", (1027, 1, 1), 9001, 3), ("deformed", (1, 35, 33), 5003, 2),
-                                            ("deformed", (40, 1, 3), 2001, 3), ("annulus", (2, 40, 14), 6001, 3),
-                                            ("annulus", (1, 24, 24), 6000, 4), ("annulus", (1, 24, 12), 3000, 5)])
+                                            ("deformed", (40, 1, 3), 2001, 3), ("ring", (1, 1030, 1), 6001, 3),
+                                            ("ring", (1, 1030, 1), 3000, 2), ("ring", (1, 300, 1), 3000, 7),
+                                            ("annulus", (2, 40, 14), 6001, 3), ("annulus", (1, 24, 12), 3000, 5)])
 def test_thin_meshes(oracle_mod, kind, shape, n, N, alpha):
     print("case thin gather", kind, shape, n, N, alpha, flush=True)
     rng = np.random.Generator(np.random.PCG64(11))
@@ -27,6 +29,13 @@ def test_thin_meshes(oracle_mod, kind, shape, n, N, alpha):
         mesh, part, species = w.mesh, w.PartState, w.species
         kw = dict(tracking=stage.TRACK_REFMAPPING, refmapping_guess=2, sf_radius=0.02, charge=w.charge, mass=w.mass,
                   mpf=w.mpf)
+    elif kind == "ring":     # curved elements; the radius reaches no periodic image in z
+        mesh = M.annulus(shape, 0.5, 0.51, 0.01, NGeo=2)
+        th, r = 2 * np.pi * rng.uniform(0.0, 1.0, n) ** 2, rng.uniform(0.5005, 0.5095, n)
+        pos = np.stack([r * np.cos(th), r * np.sin(th), rng.uniform(0.0005, 0.0095, n)], 1)
+        part = np.hstack([pos, W.maxwellian(rng, n, 2.0, stage.ELECTRON_MASS)])
+        species = np.ones(n, np.int32)
+        kw = dict(tracking=stage.TRACK_REFMAPPING, refmapping_guess=2, sf_radius=0.0006)
     else:
         hi = np.array(shape) / 8.0
         mesh = M.cartesian_box(shape, hi=tuple(hi), periodic=tuple(s >= 4 for s in shape))
